@@ -60,11 +60,44 @@ ZK_HD u64 reduce_lohi42(u64 a, u64 b)
     return r + (c ? ZK_EPS : 0);
 }
 
+// The same sum with the wrap entered as a borrow of the low word (the rare
+// case when it goes below zero) and a carry of the high word: no mask to
+// select, no zero-extended pair to build (4 instructions instead of 7).
+ZK_HD u64 reduce_lohi42_nc(u64 a, u64 b, bool &rare)
+{
+    const u64 t = (u64)(u32)(b >> 32) * ZK_EPS + a;
+    unsigned c, r;
+    const u32 hi = __builtin_addc((u32)(t >> 32), (u32)b, 0u, &c);
+    const u32 lo = __builtin_subc((u32)t, opaque_zero(), c, &r);
+    rare |= r != 0;
+    return ((u64)(hi + c) << 32) | lo;
+}
+
+// The same for a, b < 2^64 - 2^32: the multiply-add can wrap too, to at most
+// 2^64 - 2^33; each wrap is worth 2^32 - 1 and both enter as above.
+ZK_HD u64 reduce_lohi64(u64 a, u64 b, bool &rare)
+{
+    u64 t;
+#ifdef __HIP_DEVICE_COMPILE__
+    u64 k;  // carry-out of the multiply-add, as gl_reduce_small_mad_nc
+    asm("v_mad_u64_u32 %0, %1, %2, -1, %3\n\ts_nop 1" : "=v"(t), "=s"(k) : "v"((u32)(b >> 32)), "v"(a));
+    const bool c1 = __builtin_amdgcn_inverse_ballot_w64(k);
+#else
+    const bool c1 = __builtin_add_overflow((u64)(u32)(b >> 32) * ZK_EPS, a, &t);
+#endif
+    unsigned c2, r1, r2;
+    const u32 hi = __builtin_addc((u32)(t >> 32), (u32)b, (unsigned)c1, &c2);
+    u32 lo = __builtin_subc((u32)t, opaque_zero(), (unsigned)c1, &r1);
+    lo = __builtin_subc(lo, opaque_zero(), c2, &r2);
+    rare |= (r1 | r2) != 0;
+    return ((u64)(hi + c2) << 32) | lo;
+}
+
 // state <- M state + rcn (the next round's constants), M circulant (first row
 // circ) plus diag.  Row r is rcn[r] + sum of 13 products of a state element
 // with a constant below 2^6: the low and high 32-bit halves are accumulated
 // separately (the sums start at the constant's halves and stay below 2^42),
-// then reduced once by reduce_lohi42.  Inputs and outputs
+// then reduced once by reduce_lohi42_nc.  Inputs and outputs
 // are relaxed (any u64).  The coefficients come from mds_coeff:
 //
 // the MDS coefficients as multiplier operands.  The powers of two among them
@@ -85,7 +118,9 @@ ZK_HD u32 mds_coeff(int i)
     return c;
 }
 
-ZK_HD void mds_fold(u64 s[12], const u64 *rcn)
+// `need` (uniform across the wave): bit q set when rows 4q .. 4q + 3 are
+// wanted; the others are left unspecified.
+ZK_HD void mds_fold(u64 s[12], const u64 *rcn, u32 need, bool &rare)
 {
     u32 lo[12], hi[12];
 #pragma unroll
@@ -94,48 +129,211 @@ ZK_HD void mds_fold(u64 s[12], const u64 *rcn)
         hi[j] = (u32)(s[j] >> 32);
     }
 #pragma unroll
-    for (int r = 0; r < 12; r++) {
-        const u64 k = rcn[r];
-        u64 a = (u32)k, b = k >> 32;
+    for (int q = 0; q < 3; q++) {
+        if (!(need >> q & 1)) continue;
 #pragma unroll
-        for (int i = 0; i < 12; i++) {
-            const u64 c = i == 0 ? PoseidonConsts::circ[0] + PoseidonConsts::diag[r] : mds_coeff(i);
-            a += c * lo[(i + r) % 12];
-            b += c * hi[(i + r) % 12];
+        for (int r = 4 * q; r < 4 * q + 4; r++) {
+            const u64 k = rcn[r];
+            u64 a = (u32)k, b = k >> 32;
+#pragma unroll
+            for (int i = 0; i < 12; i++) {
+                const u64 c = i == 0 ? PoseidonConsts::circ[0] + PoseidonConsts::diag[r] : mds_coeff(i);
+                a += c * lo[(i + r) % 12];
+                b += c * hi[(i + r) % 12];
+            }
+            s[r] = reduce_lohi42_nc(a, b, rare);
         }
-        s[r] = reduce_lohi42(a, b);
     }
 }
 
-ZK_HD void full_round(u64 s[12], const u64 *rcn, bool &rare)
+ZK_HD void full_round(u64 s[12], const u64 *rcn, u32 need, bool &rare)
 {
 #pragma unroll
     for (int i = 0; i < 12; i++) s[i] = sbox7(s[i], rare);
-    mds_fold(s, rcn);
+    mds_fold(s, rcn, need, rare);
 }
 
-ZK_HD void partial_round(u64 s[12], const u64 *rcn, bool &rare)
+constexpr u32 kAllRows = 7;
+
+// ---- partial rounds in blocks ---------------------------------------------
+// Between two S-boxes of a partial round only element 0 is not linear, so K
+// consecutive linear layers need not be applied one by one.  A block takes the
+// state y[0..12) after an S-box layer, and with M the MDS matrix, Z the
+// projection that clears element 0 and y_i the S-box output of the block's
+// i-th inner round, the state after its j-th layer is
+//   s_j = (M Z)^(j-1) M y + sum_{i<j} (M Z)^(j-1-i) M e0 y_i,
+// a combination of 12 + j - 1 known values with non-negative coefficients.
+// Element 0 of s_1 .. s_(K-1) is all the inner S-boxes need; the other eleven
+// elements are formed once, for s_K.
+template <int K>
+struct PartialBlock {
+    static constexpr int IN = 12 + K - 1;  // y[0..12), then y_1 .. y_(K-1)
+    u64 v[K][IN];                          // row 0 of s_(j+1), j < K - 1
+    u64 f[12][IN];                         // s_K
+};
+
+template <int K>
+__host__ __device__ constexpr PartialBlock<K> make_partial_block()
 {
-    s[0] = sbox7(s[0], rare);
-    mds_fold(s, rcn);
+    PartialBlock<K> t{};
+    constexpr int IN = PartialBlock<K>::IN;
+    u64 s[12][IN] = {};  // s_0: y itself
+    for (int i = 0; i < 12; i++) s[i][i] = 1;
+    for (int j = 0; j < K; j++) {
+        if (j)  // element 0 is replaced by the inner S-box output y_j
+            for (int c = 0; c < IN; c++) s[0][c] = c == 12 + j - 1;
+        u64 n[12][IN] = {};
+        for (int r = 0; r < 12; r++)
+            for (int i = 0; i < 12; i++) {
+                const u64 m = PoseidonConsts::circ[i] + (i == 0 ? PoseidonConsts::diag[r] : 0);
+                for (int c = 0; c < IN; c++) n[r][c] += m * s[(i + r) % 12][c];
+            }
+        for (int r = 0; r < 12; r++)
+            for (int c = 0; c < IN; c++) s[r][c] = n[r][c];
+        for (int c = 0; c < IN; c++) t.v[j][c] = s[0][c];
+    }
+    for (int r = 0; r < 12; r++)
+        for (int c = 0; c < IN; c++) t.f[r][c] = s[r][c];
+    return t;
 }
 
-// 4 full rounds, 22 partial rounds (S-box on lane 0), 4 full rounds; round
-// r's constants are added by round r-1's MDS (round 0's explicitly).  The
-// round loops are not unrolled: one round body is ~1-2k instructions, so the
-// whole permutation stays resident in the instruction cache.  Input: relaxed;
-// output: relaxed (canonicalise with gl_canon).
-ZK_HD void poseidon_permute(u64 s[12], bool &rare)
+// The round constants of the partial rounds 4 .. 25 with those of elements
+// 1 .. 11 moved through the linear layers: k[r - 4] is added to element 0
+// before round r's S-box (r = 26: element 0 of the next full round), and tail
+// holds what is left for elements 1 .. 11 before round 26.
+struct PartialConsts {
+    u64 k[23];
+    u64 tail[12];
+};
+
+__host__ __device__ constexpr PartialConsts make_partial_consts()
+{
+    constexpr u64 rc[360] = ZK_POSEIDON_RC_TABLE;
+    PartialConsts t{};
+    u64 e[12] = {};
+    for (int i = 0; i < 12; i++) e[i] = rc[48 + i];
+    for (int r = 4; r < 26; r++) {
+        t.k[r - 4] = e[0];
+        e[0] = 0;
+        u64 n[12] = {};
+        for (int row = 0; row < 12; row++) {
+            unsigned __int128 acc = rc[12 * (r + 1) + row];
+            for (int i = 0; i < 12; i++)
+                acc += (unsigned __int128)(PoseidonConsts::circ[i] + (i == 0 ? PoseidonConsts::diag[row] : 0)) *
+                       e[(i + row) % 12];
+            n[row] = (u64)(acc % ZK_P);
+        }
+        for (int i = 0; i < 12; i++) e[i] = n[i];
+    }
+    t.k[22] = e[0];
+    for (int i = 1; i < 12; i++) t.tail[i] = e[i];
+    return t;
+}
+
+static __constant__ const PartialConsts kPartialConstDev = make_partial_consts();
+static const PartialConsts kPartialConstHost = make_partial_consts();
+
+ZK_HD const PartialConsts &partial_constants()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return kPartialConstDev;
+#else
+    return kPartialConstHost;
+#endif
+}
+
+// A coefficient as a multiplier operand: small ones are instruction
+// immediates, the others scalar registers; powers of two are hidden from the
+// compiler (see mds_coeff).
+template <u64 C>
+ZK_HD u32 block_coeff()
+{
+    static_assert(C < (1ull << 32), "coefficient exceeds 32 bits");
+#ifdef __HIP_DEVICE_COMPILE__
+    if constexpr (C > 1 && (C & (C - 1)) == 0) {
+        u32 r;
+        asm("s_mov_b32 %0, %1" : "=s"(r) : "i"((u32)C));
+        return r;
+    }
+#endif
+    return (u32)C;
+}
+
+// One block: s is the state after an S-box layer; k[0..K) the constants of
+// element 0 after each layer.  Returns the state before the next S-box.
+template <int K>
+ZK_HD void partial_block(u64 s[12], const u64 *k, bool &rare)
+{
+    using T = PartialBlock<K>;
+    u32 lo[T::IN], hi[T::IN];
+#pragma unroll
+    for (int i = 0; i < 12; i++) {
+        lo[i] = (u32)s[i];
+        hi[i] = (u32)(s[i] >> 32);
+    }
+    static_for<0, K - 1>([&](auto jc) {
+        constexpr int j = decltype(jc)::value;
+        u64 a = (u32)k[j], b = k[j] >> 32;
+        static_for<0, 12 + j>([&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            constexpr PartialBlock<K> tab = make_partial_block<K>();
+            a += (u64)block_coeff<tab.v[j][c]>() * lo[c];
+            b += (u64)block_coeff<tab.v[j][c]>() * hi[c];
+        });
+        const u64 y = sbox7(reduce_lohi64(a, b, rare), rare);
+        lo[12 + j] = (u32)y;
+        hi[12 + j] = (u32)(y >> 32);
+    });
+    static_for<0, 12>([&](auto rc) {
+        constexpr int r = decltype(rc)::value;
+        u64 a = r ? 0 : (u32)k[K - 1], b = r ? 0 : k[K - 1] >> 32;
+        static_for<0, T::IN>([&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            constexpr PartialBlock<K> tab = make_partial_block<K>();
+            a += (u64)block_coeff<tab.f[r][c]>() * lo[c];
+            b += (u64)block_coeff<tab.f[r][c]>() * hi[c];
+        });
+        s[r] = reduce_lohi64(a, b, rare);
+    });
+}
+
+// Layers per block.  The rate of the permutation alone with blocks of 1 (one
+// layer at a time), 2, 3 and 4 layers on an MI355X: 2.29, 2.91, 3.18 and
+// 3.26 G/s (68.8 k, 54.0 k, 49.5 k and 48.3 k SIMD-cycles per wave).  Five
+// layers would need coefficients of 37 bits, i.e. two multiply-adds more per
+// product; four reach 2^28.3, with rows whose sum is below 2^31.8, so the
+// 32-bit halves' sums stay below 2^63.8.
+constexpr int kBlock = 4;
+constexpr int kBlock0 = 3;               // layers of the first block: those of rounds 3, 4, 5
+constexpr int kBlocks = (23 - kBlock0) / kBlock;
+static_assert(kBlock0 + kBlocks * kBlock == 23, "the layers of rounds 3 .. 25");
+
+// 4 full rounds, 22 partial rounds (S-box on element 0), 4 full rounds; the
+// constants of rounds 1 .. 3 and 27 .. 29 are added by the layer before
+// (round 0's explicitly).  The layer of the fourth full round opens the first
+// block.  The loops are not unrolled, so the whole permutation stays resident
+// in the instruction cache.  Input: relaxed; output: relaxed (canonicalise
+// with gl_canon), only the rows of `need` (mds_fold).
+ZK_HD void poseidon_permute(u64 s[12], bool &rare, u32 need = kAllRows)
 {
     const u64 *rc = round_constants();
+    const PartialConsts &pc = partial_constants();
 #pragma unroll
     for (int i = 0; i < 12; i++) s[i] = gl_add_nc(s[i], rc[i], rare);
 #pragma unroll 1
-    for (int r = 0; r < 4; r++) full_round(s, rc + 12 * (r + 1), rare);
+    for (int r = 0; r < 3; r++) full_round(s, rc + 12 * (r + 1), kAllRows, rare);
+#pragma unroll
+    for (int i = 0; i < 12; i++) s[i] = sbox7(s[i], rare);
+    partial_block<kBlock0>(s, pc.k, rare);
 #pragma unroll 1
-    for (int r = 4; r < 26; r++) partial_round(s, rc + 12 * (r + 1), rare);
+    for (int b = 0; b < kBlocks; b++) {
+        s[0] = sbox7(s[0], rare);
+        partial_block<kBlock>(s, pc.k + kBlock0 + kBlock * b, rare);
+    }
+#pragma unroll
+    for (int i = 1; i < 12; i++) s[i] = gl_add_nc(s[i], pc.tail[i], rare);
 #pragma unroll 1
-    for (int r = 26; r < 30; r++) full_round(s, rc + 12 * (r + 1), rare);
+    for (int r = 26; r < 30; r++) full_round(s, rc + 12 * (r + 1), r < 29 ? kAllRows : need, rare);
 }
 
 // The same permutation with canonical arithmetic only (no rare cases): the
@@ -185,7 +383,7 @@ ZK_HD void hash_two(const u64 a[4], const u64 b[4], u64 out[4])
         s[8 + i] = 0;
     }
     bool rare = false;
-    poseidon_permute(s, rare);
+    poseidon_permute(s, rare, 1u);  // the digest is rows 0 .. 3
     if (rare) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -197,6 +395,16 @@ ZK_HD void hash_two(const u64 a[4], const u64 b[4], u64 out[4])
     }
 #pragma unroll
     for (int i = 0; i < 4; i++) out[i] = gl_canon(s[i]);
+}
+
+// The rows of the state that are read after a sponge's permutation with `rem`
+// elements left before it: the digest after the last, else the capacity and
+// the rate elements that the next chunk does not overwrite.
+ZK_HD u32 sponge_rows(u32 rem)
+{
+    if (rem <= 8) return 1u;
+    const u32 m = rem - 8;  // elements of the next chunk and after
+    return 4u | (m < 8 ? 2u : 0u) | (m < 4 ? 1u : 0u);
 }
 
 // hash_or_noop over n elements fetched by `get(i)`: n <= 4 copies the input,
@@ -223,7 +431,7 @@ ZK_HD void hash_one_chunks(Get get, u32 n, u64 out[4], Chunk chunk)
         for (u32 i = 0; i < 8; i++)
             if (i < rem) s[i] = get(idx + i);
         chunk(idx, rem < 8 ? rem : 8u, (const u64 *)s);
-        poseidon_permute(s, rare);
+        poseidon_permute(s, rare, sponge_rows(rem));
     }
     if (rare) {  // some lane hit a rare relaxed case: redo the sponge exactly
 #pragma unroll
