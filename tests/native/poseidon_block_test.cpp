@@ -1,13 +1,15 @@
 // The blocked permutation (poseidon_permute) against the exact one
 // (poseidon_permute_safe) on random and edge states, with every set of wanted
-// rows; the block reductions against 128-bit arithmetic at the limits of their
+// rows; the relaxed permutations of 16 lanes and of a quad, their lanes run in
+// lock step with the broadcasts done here; the block reductions against 128-bit arithmetic at the limits of their
 // ranges; and the block tables' row sums against the limit the 64-bit sums
 // need.  Prints "ok, N states, M rare".
 #include <cstdio>
 #include <cstdlib>
 #include <random>
 
-#include "../../zeknox_amd/csrc/poseidon.hpp"
+#include "../../zeknox_amd/csrc/poseidon_hex.hpp"
+#include "../../zeknox_amd/csrc/poseidon_quad.hpp"
 
 using namespace zk;
 typedef unsigned __int128 u128;
@@ -17,6 +19,110 @@ static int fails = 0;
 static void expect(const char *what, u64 got, u128 want)
 {
     if (gl_canon(got) != (u64)(want % ZK_P) && fails++ < 10) printf("%s: wrong value\n", what);
+}
+
+// poseidon_permute_hex_nc, lane by lane
+static void permute_hex(u64 st[12], bool &rare)
+{
+    const u64 *rc = folded_constants();
+    HexCoefs c[16];
+    u64 s[16], t[12], a[16], b[16];
+    for (u32 j = 0; j < 16; j++) {
+        hex_coefs(j, c[j]);
+        const u32 e = j < 12 ? j : j - 12;
+        s[j] = gl_add_nc(st[e], rc[e], rare);
+    }
+    auto gather = [&] {
+        for (int i = 0; i < 12; i++) t[i] = s[i];
+    };
+    auto rounds = [&](int r0, int r1) {
+        for (int r = r0; r < r1; r++) {
+            for (u32 j = 0; j < 16; j++) s[j] = hex_sbox<false>(s[j], j < 12 ? j : j - 12, r < 4 || r >= 26, rare);
+            gather();
+            for (u32 j = 0; j < 16; j++) {
+                const u64 k = rc[12 * (r + 1) + (j < 12 ? j : j - 12)];
+                u64 x = (u32)k, y = k >> 32;
+                row_sum<0>(c[j].m, t, x, y);
+                s[j] = reduce_lohi42_nc(x, y, rare);
+            }
+        }
+    };
+    rounds(0, kBlockStart);
+    for (int blk = 0; blk < kBlocks; blk++) {
+        const u64 *kp = rc + 12 * (kBlockStart + 1 + kBlock * blk);
+        gather();
+        const u64 y0 = sbox7(t[0], rare);
+        for (u32 j = 0; j < 16; j++) {
+            const u64 k = j >= 12 && j < 15 ? kp[12 * (j - 12)] : (j == 0 ? kp[36] : 0);
+            a[j] = (u32)k;
+            b[j] = k >> 32;
+            row_sum<1>(c[j].b, t, a[j], b[j]);
+            row_add(c[j].b[0], y0, a[j], b[j]);
+        }
+        for (int q = 0; q < kBlock - 1; q++) {
+            u64 v[16];
+            for (u32 j = 0; j < 16; j++) v[j] = reduce_lohi64(a[j], b[j], rare);
+            const u64 y = sbox7(v[12 + q], rare);
+            for (u32 j = 0; j < 16; j++) row_add(c[j].b[12 + q], y, a[j], b[j]);
+        }
+        for (u32 j = 0; j < 16; j++) s[j] = reduce_lohi64(a[j], b[j], rare);
+    }
+    for (u32 e = 1; e < 12; e++) s[e] = gl_add_nc(s[e], rc[12 * 26 + e], rare);
+    rounds(26, 30);
+    for (int e = 0; e < 12; e++) st[e] = s[e];
+}
+
+// poseidon_permute_quad_nc, lane by lane
+static void permute_quad(u64 st[12], bool &rare)
+{
+    const u64 *rc = folded_constants();
+    QuadCoefs c[4];
+    u64 s[4][3];
+    for (u32 j = 0; j < 4; j++) {
+        quad_coefs(j, c[j]);
+        for (u32 k = 0; k < 3; k++) s[j][k] = gl_add_nc(st[3 * j + k], rc[3 * j + k], rare);
+    }
+    auto rounds = [&](int r0, int r1) {
+        for (int r = r0; r < r1; r++) {
+            for (u32 j = 0; j < 4; j++) quad_sbox<false>(s[j], j, r < 4 || r >= 26, rare);
+            u64 n[4][3];
+            for (u32 j = 0; j < 4; j++) {
+                u64 t[12];
+                for (u32 e = 0; e < 12; e++) t[e] = s[(3 * j + e) % 12 / 3][(3 * j + e) % 3];
+                quad_mds<false>(t, j, rc + 12 * (r + 1) + 3 * j, n[j]);
+            }
+            for (u32 j = 0; j < 4; j++)
+                for (int k = 0; k < 3; k++) s[j][k] = n[j][k];
+        }
+    };
+    rounds(0, kBlockStart);
+    for (int blk = 0; blk < kBlocks; blk++) {
+        const u64 *kp = rc + 12 * (kBlockStart + 1 + kBlock * blk);
+        u64 t[12], a[4][4], b[4][4];  // [lane][three rows, inner value]
+        for (u32 e = 0; e < 12; e++) t[e] = s[e / 3][e % 3];
+        const u64 y0 = sbox7(t[0], rare);
+        for (u32 j = 0; j < 4; j++)
+            for (int k = 0; k < 4; k++) {
+                const u32 *cc = k < 3 ? c[j].f[k] : c[j].v;
+                const u64 kk = k == 3 ? kp[12 * j] : (j + k == 0 ? kp[36] : 0);
+                a[j][k] = (u32)kk;
+                b[j][k] = kk >> 32;
+                row_sum<1>(cc, t, a[j][k], b[j][k]);
+                row_add(cc[0], y0, a[j][k], b[j][k]);
+            }
+        for (int q = 0; q < kBlock - 1; q++) {
+            const u64 y = sbox7(reduce_lohi64(a[q][3], b[q][3], rare), rare);
+            for (u32 j = 0; j < 4; j++) {
+                row_add(c[j].v[12 + q], y, a[j][3], b[j][3]);
+                for (int k = 0; k < 3; k++) row_add(c[j].f[k][12 + q], y, a[j][k], b[j][k]);
+            }
+        }
+        for (u32 j = 0; j < 4; j++)
+            for (int k = 0; k < 3; k++) s[j][k] = reduce_lohi64(a[j][k], b[j][k], rare);
+    }
+    for (u32 e = 1; e < 12; e++) s[e / 3][e % 3] = gl_add_nc(s[e / 3][e % 3], rc[12 * 26 + e], rare);
+    rounds(26, 30);
+    for (u32 e = 0; e < 12; e++) st[e] = s[e / 3][e % 3];
 }
 
 template <int K>
@@ -43,6 +149,19 @@ int main(int argc, char **argv)
         u64 in[12], want[12];
         for (int i = 0; i < 12; i++) want[i] = in[i] = it % 3 ? g() : edges[g() % 10];
         poseidon_permute_safe(want);
+        for (int lanes = 0; lanes < 2; lanes++) {
+            u64 s[12];
+            for (int i = 0; i < 12; i++) s[i] = in[i];
+            bool rare = false;
+            lanes ? permute_quad(s, rare) : permute_hex(s, rare);
+            if (rare) {
+                rares++;
+                continue;
+            }
+            for (int i = 0; i < 12; i++)
+                if (gl_canon(s[i]) != want[i] && fails++ < 10)
+                    printf("state %d %s: element %d differs\n", it, lanes ? "quad" : "hex", i);
+        }
         for (u32 need = 1; need < 8; need++) {
             u64 s[12];
             for (int i = 0; i < 12; i++) s[i] = in[i];

@@ -18,16 +18,16 @@
 
 namespace zk {
 
-constexpr int kLeafThreads = 128;  // threads per workgroup of the leaf kernels
-constexpr int kNodeThreads = 128;  // threads per workgroup of the level kernels
+constexpr int kLeafThreads = 128;  // threads per workgroup of the forests' leaf kernels
+constexpr int kNodeThreads = 128;  // threads per workgroup of the forests' level kernels
 // Levels with at most this many nodes (all subtrees) use a quad of lanes per
-// node.
+// node: 36 us at 2^16 nodes against 39 with one lane; at 2^17 one lane takes
+// 53 us, a quad 70.
 constexpr u64 kQuadMaxNodes = 1u << 16;
-// Levels with at most this many nodes use 16 lanes per node: 14-17 us per
-// level against 20 us with a quad (2^11-2^12 nodes; each lane does one S-box
-// and one MDS row per round, against three of each, plus a lane exchange per
-// element; 4/3 the work of a quad, so wider levels keep the quad).
-constexpr u64 kHexMaxNodes = 1u << 12;
+// Levels with at most this many nodes use 16 lanes per node: 11 us at 2^13
+// nodes against 13 with a quad, 7.7 at 2^12; at 2^14 a quad takes 13 us, 16
+// lanes 20.
+constexpr u64 kHexMaxNodes = 1u << 13;
 // Workgroups of one forest launch at most (HIP counts a grid in threads, as a
 // 32-bit number); a longer launch is split, each part with its own table.
 constexpr u64 kForestMaxBlocks = 1ull << 23;

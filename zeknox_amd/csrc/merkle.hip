@@ -24,8 +24,22 @@
 
 namespace zk {
 
-// Trees with at most this many leaves use a quad of lanes per leaf.
-constexpr u64 kQuadMaxLeaves = 1u << 15;
+// Lanes per leaf by the number of leaves, where one form's time per
+// permutation passes the other's on an MI355X (1024 SIMDs): 16 lanes up to
+// 2^13 leaves (two waves per SIMD: 10.9 us; a quad 13.1), a quad up to 2^16
+// (19 us at 2^15, 36 at 2^16; one lane 39 at either), then one lane (53 us at
+// 2^17, where a quad takes 70).
+constexpr u64 kHexMaxLeaves = 1u << 13;
+constexpr u64 kQuadMaxLeaves = 1u << 16;
+
+// Threads per workgroup of one tree's kernels.  One lane per leaf: four waves,
+// one for each SIMD of a CU; with two, 2^17 leaves (two waves per SIMD) were
+// placed unevenly and took 300 us instead of 235 (32 elements), at 2^20 leaves
+// there is no difference.  Several lanes per hash and levels, often less than
+// a wave per SIMD: one wave, which spreads evenly (2^12 leaves of 135 elements
+// with 16 lanes each: 199 -> 153 us).
+constexpr int kTreeLeafThreads = 256;
+constexpr int kTreeNodeThreads = 64;
 
 static u32 ilog2(u64 x)
 {
@@ -91,12 +105,16 @@ __device__ __forceinline__ void leaf_hash_thread(const LeafArgs &a, u64 t, u64 *
     for (int k = 0; k < 4; k++) o[k] = h[k];
 }
 
-// At least four waves per SIMD: the leaf-row variant fits in 111 VGPRs.
+// Exactly four waves per SIMD (102 VGPRs would allow it, 92 to 98 five): a
+// power of two of leaves then runs in whole rounds.  2^20 leaves of 135
+// elements take 5.7 ms; where the compiler found registers for five waves, the
+// fourth round ran on a fifth of the slots and they took 6.4 ms.
 template <LeafLayout LAYOUT, bool ROWS>
-__global__ __launch_bounds__(kLeafThreads, 4) void leaf_hash_kernel(LeafArgs a)
+__global__ __launch_bounds__(kTreeLeafThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void leaf_hash_kernel(
+    LeafArgs a)
 {
-    __shared__ u64 ring[ROWS ? kLeafThreads * kRowRingPitch : 1];
-    leaf_hash_thread<LAYOUT, ROWS>(a, (u64)blockIdx.x * kLeafThreads + threadIdx.x, ring);
+    __shared__ u64 ring[ROWS ? kTreeLeafThreads * kRowRingPitch : 1];
+    leaf_hash_thread<LAYOUT, ROWS>(a, (u64)blockIdx.x * kTreeLeafThreads + threadIdx.x, ring);
 }
 
 // The leaves of many commits in one launch (batched commits): workgroup b
@@ -116,17 +134,19 @@ __global__ __launch_bounds__(kLeafThreads, 4) void leaf_hash_forest_kernel(const
 // the GPU with one lane per leaf (a third of the latency).  Lanes past the
 // last leaf hash leaf 0 again and store nothing.
 template <LeafLayout LAYOUT, bool ROWS>
-__global__ __launch_bounds__(kLeafThreads) void leaf_hash_quad_kernel(LeafArgs a)
+__global__ __launch_bounds__(kTreeNodeThreads) void leaf_hash_quad_kernel(LeafArgs a)
 {
-    const u64 t = ((u64)blockIdx.x * kLeafThreads + threadIdx.x) >> 2;
+    const u64 t = ((u64)blockIdx.x * kTreeNodeThreads + threadIdx.x) >> 2;
     const u32 j = threadIdx.x & 3;
     const bool ok = t < a.n_leaves;
     const u64 tc = ok ? t : 0;
+    QuadCoefs c;
+    quad_coefs(j, c);
     u64 leaf, h[3];
     if constexpr (LAYOUT == LeafLayout::RowMajor) {
         leaf = tc;
         const u64 *p = a.leaves + leaf * a.leaf_size;
-        hash_one_quad([p](u32 i) { return p[i]; }, a.leaf_size, j, h);
+        hash_one_quad([p](u32 i) { return p[i]; }, a.leaf_size, j, c, h);
     } else {
         leaf = zk_bitrev((u32)tc, a.lg_leaves);
         const u64 *p = a.leaves + tc;
@@ -138,9 +158,9 @@ __global__ __launch_bounds__(kLeafThreads) void leaf_hash_quad_kernel(LeafArgs a
                 const u64 v = p[(u64)i * cs];
                 if (w) q[i] = v;
                 return v;
-            }, a.leaf_size, j, h);
+            }, a.leaf_size, j, c, h);
         } else {
-            hash_one_quad([p, cs](u32 i) { return p[(u64)i * cs]; }, a.leaf_size, j, h);
+            hash_one_quad([p, cs](u32 i) { return p[(u64)i * cs]; }, a.leaf_size, j, c, h);
         }
     }
     if (!ok) return;
@@ -159,10 +179,47 @@ __global__ __launch_bounds__(kLeafThreads) void leaf_hash_quad_kernel(LeafArgs a
     }
 }
 
-// One level: 2^r nodes per subtree starting at `base`.
-__global__ __launch_bounds__(kNodeThreads) void level_hash_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub, u64 D)
+// Leaf hashing with 16 lanes per leaf, for the smallest trees.  Groups past
+// the last leaf hash leaf 0 again and store nothing.
+template <LeafLayout LAYOUT, bool ROWS>
+__global__ __launch_bounds__(kTreeNodeThreads) void leaf_hash_hex_kernel(LeafArgs a)
 {
-    const u64 t = (u64)blockIdx.x * kNodeThreads + threadIdx.x;
+    const u64 t = ((u64)blockIdx.x * kTreeNodeThreads + threadIdx.x) >> 4;
+    const u32 j = threadIdx.x & 15, lb = threadIdx.x & 48;
+    const bool ok = t < a.n_leaves;
+    const u64 tc = ok ? t : 0;
+    HexCoefs c;
+    hex_coefs(j, c);
+    u64 leaf, h;
+    if constexpr (LAYOUT == LeafLayout::RowMajor) {
+        leaf = tc;
+        const u64 *p = a.leaves + leaf * a.leaf_size;
+        h = hash_one_hex([p](u32 i) { return p[i]; }, a.leaf_size, j, lb, c);
+    } else {
+        leaf = zk_bitrev((u32)tc, a.lg_leaves);
+        const u64 *p = a.leaves + tc;
+        const u64 cs = a.col_stride;
+        u64 *q = ROWS ? a.rows + leaf * a.leaf_size : nullptr;
+        const bool w = ROWS && ok;
+        h = hash_one_hex([p, cs, q, w](u32 i) {
+            const u64 v = p[(u64)i * cs];
+            if (w) q[i] = v;
+            return v;
+        }, a.leaf_size, j, lb, c);
+    }
+    if (!ok || j >= 4) return;
+    u64 slot = leaf;
+    if (a.sub_leaves) {
+        const u64 s = leaf / a.sub_leaves, i = leaf % a.sub_leaves;
+        slot = s * a.sub_digests + (a.sub_digests - a.sub_leaves) + i;
+    }
+    a.out[slot * 4 + j] = h;
+}
+
+// One level: 2^r nodes per subtree starting at `base`.
+__global__ __launch_bounds__(kTreeNodeThreads) void level_hash_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub, u64 D)
+{
+    const u64 t = (u64)blockIdx.x * kTreeNodeThreads + threadIdx.x;
     if (t >= nodes * n_sub) return;
     const u64 s = t / nodes, node = base + t % nodes;
     u64 *sd = d + s * D * 4;
@@ -180,17 +237,19 @@ __global__ __launch_bounds__(kNodeThreads) void level_hash_kernel(u64 *d, u64 no
 // One level with a quad of lanes per node (levels too small to fill the GPU
 // with one lane per node: a third of the latency).  Lanes past the last node
 // hash node 0 again and store nothing, so every quad stays complete.
-__global__ __launch_bounds__(kNodeThreads) void level_hash_quad_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub,
+__global__ __launch_bounds__(kTreeNodeThreads) void level_hash_quad_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub,
                                                                        u64 D)
 {
-    const u64 t = (u64)blockIdx.x * kNodeThreads + threadIdx.x;
+    const u64 t = (u64)blockIdx.x * kTreeNodeThreads + threadIdx.x;
     const u32 j = threadIdx.x & 3;
     const u64 total = nodes * n_sub, x = t >> 2;
     const u64 xc = x < total ? x : 0;
     const u64 s = xc / nodes, node = base + xc % nodes;
     u64 *sd = d + s * D * 4;
+    QuadCoefs c;
+    quad_coefs(j, c);
     u64 out[3];
-    hash_two_quad(sd + (2 * node + 2) * 4, sd + (2 * node + 3) * 4, j, out);
+    hash_two_quad(sd + (2 * node + 2) * 4, sd + (2 * node + 3) * 4, j, c, out);
     if (x < total) {
         u64 *o = sd + node * 4;
         if (j == 0) {
@@ -206,16 +265,18 @@ __global__ __launch_bounds__(kNodeThreads) void level_hash_quad_kernel(u64 *d, u
 // One level with 16 lanes per node (hash_two_hex), for levels whose latency
 // rather than their work bounds them.  Groups past the last node hash node 0
 // again and store nothing, so every group stays complete.
-__global__ __launch_bounds__(kNodeThreads) void level_hash_hex_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub,
+__global__ __launch_bounds__(kTreeNodeThreads) void level_hash_hex_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub,
                                                                       u64 D)
 {
-    const u64 t = (u64)blockIdx.x * kNodeThreads + threadIdx.x;
+    const u64 t = (u64)blockIdx.x * kTreeNodeThreads + threadIdx.x;
     const u32 j = threadIdx.x & 15, lb = threadIdx.x & 48;  // lane in the group, group's first wave lane
     const u64 total = nodes * n_sub, x = t >> 4;
     const u64 xc = x < total ? x : 0;
     const u64 s = xc / nodes, node = base + xc % nodes;
     u64 *sd = d + s * D * 4;
-    const u64 out = hash_two_hex(sd + (2 * node + 2) * 4, sd + (2 * node + 3) * 4, j, lb);
+    HexCoefs c;
+    hex_coefs(j, c);
+    const u64 out = hash_two_hex(sd + (2 * node + 2) * 4, sd + (2 * node + 3) * 4, j, lb, c);
     if (x < total && j < 4) sd[node * 4 + j] = out;
 }
 
@@ -248,8 +309,10 @@ __global__ __launch_bounds__(kNodeThreads) void level_hash_forest_kernel(const F
         for (int k = 0; k < 4; k++) o[k] = h[k];
     } else if constexpr (G == 4) {
         const u32 j = threadIdx.x & 3;
+        QuadCoefs c;
+        quad_coefs(j, c);
         u64 out[3];
-        hash_two_quad(ca, cb, j, out);
+        hash_two_quad(ca, cb, j, c, out);
         if (ok) {
             if (j == 0) {
                 o[0] = out[0];
@@ -262,7 +325,9 @@ __global__ __launch_bounds__(kNodeThreads) void level_hash_forest_kernel(const F
     } else {
         static_assert(G == 16, "1, 4 or 16 lanes per node");
         const u32 j = threadIdx.x & 15, lb = threadIdx.x & 48;
-        const u64 h = hash_two_hex(ca, cb, j, lb);
+        HexCoefs c;
+        hex_coefs(j, c);
+        const u64 h = hash_two_hex(ca, cb, j, lb, c);
         if (ok && j < 4) o[j] = h;
     }
 }
@@ -285,11 +350,13 @@ __global__ __launch_bounds__(16 * kTopNodes) void tree_top_kernel(u64 *d, u64 *c
     __syncthreads();
     const u32 j = threadIdx.x & 15, q = threadIdx.x >> 4, lb = threadIdx.x & 48;
     const u32 wave_q0 = q & ~3u;  // the wave's first group
+    HexCoefs c;
+    hex_coefs(j, c);
     u64 *cur = bufA, *nxt = bufB;
     for (u32 nodes = m; nodes >= 2; nodes >>= 1) {
         if (wave_q0 < nodes) {  // uniform across the wave
             const u32 qc = q < nodes ? q : 0;
-            const u64 h = hash_two_hex(cur + 8 * qc, cur + 8 * qc + 4, j, lb);
+            const u64 h = hash_two_hex(cur + 8 * qc, cur + 8 * qc + 4, j, lb, c);
             if (q < nodes && j < 4) {
                 sd[(u64)(nodes - 2 + q) * 4 + j] = h;
                 nxt[4 * q + j] = h;
@@ -301,7 +368,7 @@ __global__ __launch_bounds__(16 * kTopNodes) void tree_top_kernel(u64 *d, u64 *c
         nxt = tmp;
     }
     if (wave_q0 == 0) {
-        const u64 h = hash_two_hex(cur, cur + 4, j, lb);
+        const u64 h = hash_two_hex(cur, cur + 4, j, lb, c);
         if (q == 0 && j < 4) caps[(u64)blockIdx.x * 4 + j] = h;
     }
 }
@@ -309,9 +376,9 @@ __global__ __launch_bounds__(16 * kTopNodes) void tree_top_kernel(u64 *d, u64 *c
 // ----------------------------------------------------------------- other hashers
 // Keccak and Poseidon2 trees: one lane per leaf / node / cap entry.
 template <LeafLayout LAYOUT, typename H>
-__global__ __launch_bounds__(kLeafThreads) void leaf_hash_h_kernel(LeafArgs a)
+__global__ __launch_bounds__(kTreeNodeThreads) void leaf_hash_h_kernel(LeafArgs a)
 {
-    const u64 t = (u64)blockIdx.x * kLeafThreads + threadIdx.x;
+    const u64 t = (u64)blockIdx.x * kTreeNodeThreads + threadIdx.x;
     if (t >= a.n_leaves) return;
     u64 leaf, h[4];
     if constexpr (LAYOUT == LeafLayout::RowMajor) {
@@ -332,9 +399,9 @@ __global__ __launch_bounds__(kLeafThreads) void leaf_hash_h_kernel(LeafArgs a)
 }
 
 template <typename H>
-__global__ __launch_bounds__(kNodeThreads) void level_hash_h_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub, u64 D)
+__global__ __launch_bounds__(kTreeNodeThreads) void level_hash_h_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub, u64 D)
 {
-    const u64 t = (u64)blockIdx.x * kNodeThreads + threadIdx.x;
+    const u64 t = (u64)blockIdx.x * kTreeNodeThreads + threadIdx.x;
     if (t >= nodes * n_sub) return;
     const u64 s = t / nodes, node = base + t % nodes;
     u64 *sd = d + s * D * 4;
@@ -350,9 +417,9 @@ __global__ __launch_bounds__(kNodeThreads) void level_hash_h_kernel(u64 *d, u64 
 }
 
 template <typename H>
-__global__ __launch_bounds__(kNodeThreads) void cap_hash_h_kernel(u64 *caps, const u64 *d, u64 n_caps, u64 D)
+__global__ __launch_bounds__(kTreeNodeThreads) void cap_hash_h_kernel(u64 *caps, const u64 *d, u64 n_caps, u64 D)
 {
-    const u64 s = (u64)blockIdx.x * kNodeThreads + threadIdx.x;
+    const u64 s = (u64)blockIdx.x * kTreeNodeThreads + threadIdx.x;
     if (s >= n_caps) return;
     const u64 *sd = d + s * D * 4;
     u64 l[4], r[4], o[4];
@@ -421,30 +488,29 @@ void merkle_launch(const TreeShape &t, u64 *digests, u64 *caps, const u64 *leave
         a.sub_leaves = L;
         a.sub_digests = D;
     }
-    const u32 nb = blocks_for(t.n_leaves, kLeafThreads);
-    if (t.n_leaves <= kQuadMaxLeaves && t.leaf_size > 4) {
-        ProfScope ps(layout == LeafLayout::RowMajor ? "merkle.leaves" : "merkle.leaves_colmajor", st);
-        const u32 nq = blocks_for(4 * t.n_leaves, kLeafThreads);
-        if (layout == LeafLayout::RowMajor)
-            hipLaunchKernelGGL((leaf_hash_quad_kernel<LeafLayout::RowMajor, false>), dim3(nq), dim3(kLeafThreads), 0,
-                               st, a);
-        else if (a.rows)
-            hipLaunchKernelGGL((leaf_hash_quad_kernel<LeafLayout::ColMajorRev, true>), dim3(nq), dim3(kLeafThreads),
-                               0, st, a);
-        else
-            hipLaunchKernelGGL((leaf_hash_quad_kernel<LeafLayout::ColMajorRev, false>), dim3(nq),
-                               dim3(kLeafThreads), 0, st, a);
+    {
+        const bool row_major = layout == LeafLayout::RowMajor;
+        ProfScope ps(row_major ? "merkle.leaves" : "merkle.leaves_colmajor", st);
+        // lanes per leaf; leaves of at most four elements are copied
+        const u64 lanes = t.leaf_size <= 4 || t.n_leaves > kQuadMaxLeaves ? 1 : (t.n_leaves > kHexMaxLeaves ? 4 : 16);
+        const int threads = lanes == 1 ? kTreeLeafThreads : kTreeNodeThreads;
+        const dim3 grid(blocks_for(lanes * t.n_leaves, threads)), block(threads);
+#define ZK_LEAVES(kernel)                                                                                   \
+    if (row_major)                                                                                          \
+        hipLaunchKernelGGL((kernel<LeafLayout::RowMajor, false>), grid, block, 0, st, a);                   \
+    else if (a.rows)                                                                                        \
+        hipLaunchKernelGGL((kernel<LeafLayout::ColMajorRev, true>), grid, block, 0, st, a);                 \
+    else                                                                                                    \
+        hipLaunchKernelGGL((kernel<LeafLayout::ColMajorRev, false>), grid, block, 0, st, a);
+        if (lanes == 1) {
+            ZK_LEAVES(leaf_hash_kernel)
+        } else if (lanes == 4) {
+            ZK_LEAVES(leaf_hash_quad_kernel)
+        } else {
+            ZK_LEAVES(leaf_hash_hex_kernel)
+        }
+#undef ZK_LEAVES
         ZK_HIP(hipGetLastError());
-    } else {
-    ProfScope ps(layout == LeafLayout::RowMajor ? "merkle.leaves" : "merkle.leaves_colmajor", st);
-    if (layout == LeafLayout::RowMajor)
-        hipLaunchKernelGGL((leaf_hash_kernel<LeafLayout::RowMajor, false>), dim3(nb), dim3(kLeafThreads), 0, st, a);
-    else if (a.rows)
-        hipLaunchKernelGGL((leaf_hash_kernel<LeafLayout::ColMajorRev, true>), dim3(nb), dim3(kLeafThreads), 0, st, a);
-    else
-        hipLaunchKernelGGL((leaf_hash_kernel<LeafLayout::ColMajorRev, false>), dim3(nb), dim3(kLeafThreads), 0, st,
-                           a);
-    ZK_HIP(hipGetLastError());
     }
     if (nc == t.n_leaves) return;
     // Levels wider than the top kernel's: one lane per node while the level
@@ -455,13 +521,13 @@ void merkle_launch(const TreeShape &t, u64 *digests, u64 *caps, const u64 *leave
         const u64 total = nodes * nc;
         ProfScope ps("merkle.levels", st);
         if (total > kQuadMaxNodes)
-            hipLaunchKernelGGL(level_hash_kernel, dim3(blocks_for(total, kNodeThreads)), dim3(kNodeThreads), 0, st,
+            hipLaunchKernelGGL(level_hash_kernel, dim3(blocks_for(total, kTreeNodeThreads)), dim3(kTreeNodeThreads), 0, st,
                                digests, nodes, nodes - 2, nc, D);
         else if (total > kHexMaxNodes)
-            hipLaunchKernelGGL(level_hash_quad_kernel, dim3(blocks_for(4 * total, kNodeThreads)), dim3(kNodeThreads),
+            hipLaunchKernelGGL(level_hash_quad_kernel, dim3(blocks_for(4 * total, kTreeNodeThreads)), dim3(kTreeNodeThreads),
                                0, st, digests, nodes, nodes - 2, nc, D);
         else
-            hipLaunchKernelGGL(level_hash_hex_kernel, dim3(blocks_for(16 * total, kNodeThreads)), dim3(kNodeThreads),
+            hipLaunchKernelGGL(level_hash_hex_kernel, dim3(blocks_for(16 * total, kTreeNodeThreads)), dim3(kTreeNodeThreads),
                                0, st, digests, nodes, nodes - 2, nc, D);
         ZK_HIP(hipGetLastError());
     }
@@ -540,19 +606,19 @@ static void merkle_launch_h(const TreeShape &t, u64 *digests, u64 *caps, const u
     a.out = nc == t.n_leaves ? caps : digests;
     a.sub_leaves = (nc == t.n_leaves || L == 2) ? 0 : L;
     a.sub_digests = D;
-    const u32 nb = blocks_for(t.n_leaves, kLeafThreads);
+    const u32 nb = blocks_for(t.n_leaves, kTreeNodeThreads);
     if (layout == LeafLayout::RowMajor)
-        hipLaunchKernelGGL((leaf_hash_h_kernel<LeafLayout::RowMajor, H>), dim3(nb), dim3(kLeafThreads), 0, st, a);
+        hipLaunchKernelGGL((leaf_hash_h_kernel<LeafLayout::RowMajor, H>), dim3(nb), dim3(kTreeNodeThreads), 0, st, a);
     else
-        hipLaunchKernelGGL((leaf_hash_h_kernel<LeafLayout::ColMajorRev, H>), dim3(nb), dim3(kLeafThreads), 0, st, a);
+        hipLaunchKernelGGL((leaf_hash_h_kernel<LeafLayout::ColMajorRev, H>), dim3(nb), dim3(kTreeNodeThreads), 0, st, a);
     ZK_HIP(hipGetLastError());
     if (nc == t.n_leaves) return;
     for (u64 nodes = L / 2; nodes >= 2; nodes /= 2) {
-        hipLaunchKernelGGL(level_hash_h_kernel<H>, dim3(blocks_for(nodes * nc, kNodeThreads)), dim3(kNodeThreads), 0,
+        hipLaunchKernelGGL(level_hash_h_kernel<H>, dim3(blocks_for(nodes * nc, kTreeNodeThreads)), dim3(kTreeNodeThreads), 0,
                            st, digests, nodes, nodes - 2, nc, D);
         ZK_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(cap_hash_h_kernel<H>, dim3(blocks_for(nc, kNodeThreads)), dim3(kNodeThreads), 0, st, caps,
+    hipLaunchKernelGGL(cap_hash_h_kernel<H>, dim3(blocks_for(nc, kTreeNodeThreads)), dim3(kTreeNodeThreads), 0, st, caps,
                        (const u64 *)digests, nc, D);
     ZK_HIP(hipGetLastError());
 }

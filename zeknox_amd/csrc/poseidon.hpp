@@ -197,23 +197,24 @@ __host__ __device__ constexpr PartialBlock<K> make_partial_block()
     return t;
 }
 
-// The round constants of the partial rounds 4 .. 25 with those of elements
-// 1 .. 11 moved through the linear layers: k[r - 4] is added to element 0
-// before round r's S-box (r = 26: element 0 of the next full round), and tail
-// holds what is left for elements 1 .. 11 before round 26.
-struct PartialConsts {
-    u64 k[23];
-    u64 tail[12];
+// The round constants with those of elements 1 .. 11 in the partial rounds
+// moved through the linear layers: rows 4 .. 25 keep only element 0, what is
+// left joins row 26.  Row 30 (zeros) follows the last round.
+struct FoldedConsts {
+    u64 rc[31 * 12];
 };
 
-__host__ __device__ constexpr PartialConsts make_partial_consts()
+__host__ __device__ constexpr FoldedConsts make_folded_consts()
 {
     constexpr u64 rc[360] = ZK_POSEIDON_RC_TABLE;
-    PartialConsts t{};
+    FoldedConsts t{};
+    for (int i = 0; i < 360; i++)
+        if (i < 60 || i >= 12 * 27) t.rc[i] = rc[i];
     u64 e[12] = {};
     for (int i = 0; i < 12; i++) e[i] = rc[48 + i];
     for (int r = 4; r < 26; r++) {
-        t.k[r - 4] = e[0];
+        t.rc[12 * r] = e[0];
+        for (int i = 1; i < 12; i++) t.rc[12 * r + i] = 0;
         e[0] = 0;
         u64 n[12] = {};
         for (int row = 0; row < 12; row++) {
@@ -225,20 +226,19 @@ __host__ __device__ constexpr PartialConsts make_partial_consts()
         }
         for (int i = 0; i < 12; i++) e[i] = n[i];
     }
-    t.k[22] = e[0];
-    for (int i = 1; i < 12; i++) t.tail[i] = e[i];
+    for (int i = 0; i < 12; i++) t.rc[12 * 26 + i] = e[i];
     return t;
 }
 
-static __constant__ const PartialConsts kPartialConstDev = make_partial_consts();
-static const PartialConsts kPartialConstHost = make_partial_consts();
+static __constant__ const FoldedConsts kFoldedConstDev = make_folded_consts();
+static const FoldedConsts kFoldedConstHost = make_folded_consts();
 
-ZK_HD const PartialConsts &partial_constants()
+ZK_HD const u64 *folded_constants()
 {
 #ifdef __HIP_DEVICE_COMPILE__
-    return kPartialConstDev;
+    return kFoldedConstDev.rc;
 #else
-    return kPartialConstHost;
+    return kFoldedConstHost.rc;
 #endif
 }
 
@@ -259,8 +259,9 @@ ZK_HD u32 block_coeff()
     return (u32)C;
 }
 
-// One block: s is the state after an S-box layer; k[0..K) the constants of
-// element 0 after each layer.  Returns the state before the next S-box.
+// One block: s is the state after an S-box layer; k (folded constants) row j
+// holds the constant of element 0 after layer j.  Returns the state before
+// the next S-box.
 template <int K>
 ZK_HD void partial_block(u64 s[12], const u64 *k, bool &rare)
 {
@@ -273,7 +274,7 @@ ZK_HD void partial_block(u64 s[12], const u64 *k, bool &rare)
     }
     static_for<0, K - 1>([&](auto jc) {
         constexpr int j = decltype(jc)::value;
-        u64 a = (u32)k[j], b = k[j] >> 32;
+        u64 a = (u32)k[12 * j], b = k[12 * j] >> 32;
         static_for<0, 12 + j>([&](auto cc) {
             constexpr int c = decltype(cc)::value;
             constexpr PartialBlock<K> tab = make_partial_block<K>();
@@ -286,7 +287,7 @@ ZK_HD void partial_block(u64 s[12], const u64 *k, bool &rare)
     });
     static_for<0, 12>([&](auto rc) {
         constexpr int r = decltype(rc)::value;
-        u64 a = r ? 0 : (u32)k[K - 1], b = r ? 0 : k[K - 1] >> 32;
+        u64 a = r ? 0 : (u32)k[12 * (K - 1)], b = r ? 0 : k[12 * (K - 1)] >> 32;
         static_for<0, T::IN>([&](auto cc) {
             constexpr int c = decltype(cc)::value;
             constexpr PartialBlock<K> tab = make_partial_block<K>();
@@ -305,7 +306,8 @@ ZK_HD void partial_block(u64 s[12], const u64 *k, bool &rare)
 // 32-bit halves' sums stay below 2^63.8.
 constexpr int kBlock = 4;
 constexpr int kBlock0 = 3;               // layers of the first block: those of rounds 3, 4, 5
-constexpr int kBlocks = (23 - kBlock0) / kBlock;
+constexpr int kBlocks = (23 - kBlock0) / kBlock;  // the others': from round kBlockStart on
+constexpr int kBlockStart = 3 + kBlock0;
 static_assert(kBlock0 + kBlocks * kBlock == 23, "the layers of rounds 3 .. 25");
 
 // 4 full rounds, 22 partial rounds (S-box on element 0), 4 full rounds; the
@@ -316,24 +318,75 @@ static_assert(kBlock0 + kBlocks * kBlock == 23, "the layers of rounds 3 .. 25");
 // with gl_canon), only the rows of `need` (mds_fold).
 ZK_HD void poseidon_permute(u64 s[12], bool &rare, u32 need = kAllRows)
 {
-    const u64 *rc = round_constants();
-    const PartialConsts &pc = partial_constants();
+    const u64 *rc = folded_constants();
 #pragma unroll
     for (int i = 0; i < 12; i++) s[i] = gl_add_nc(s[i], rc[i], rare);
 #pragma unroll 1
     for (int r = 0; r < 3; r++) full_round(s, rc + 12 * (r + 1), kAllRows, rare);
 #pragma unroll
     for (int i = 0; i < 12; i++) s[i] = sbox7(s[i], rare);
-    partial_block<kBlock0>(s, pc.k, rare);
+    partial_block<kBlock0>(s, rc + 12 * 4, rare);
 #pragma unroll 1
     for (int b = 0; b < kBlocks; b++) {
         s[0] = sbox7(s[0], rare);
-        partial_block<kBlock>(s, pc.k + kBlock0 + kBlock * b, rare);
+        partial_block<kBlock>(s, rc + 12 * (4 + kBlock0 + kBlock * b), rare);
     }
 #pragma unroll
-    for (int i = 1; i < 12; i++) s[i] = gl_add_nc(s[i], pc.tail[i], rare);
+    for (int i = 1; i < 12; i++) s[i] = gl_add_nc(s[i], rc[12 * 26 + i], rare);
 #pragma unroll 1
     for (int r = 26; r < 30; r++) full_round(s, rc + 12 * (r + 1), r < 29 ? kAllRows : need, rare);
+}
+
+// Coefficient rows of the lane-parallel forms (poseidon_quad.hpp,
+// poseidon_hex.hpp).  block: rows 0 .. 11 the elements after a block of kBlock
+// layers, rows 12 .. 14 element 0 after its first three; columns the 15
+// inputs.  mds: row r of one layer (rows 12 .. 15 repeat 0 .. 3).
+struct LaneRows {
+    u32 block[16][16], mds[16][12];
+};
+
+__host__ __device__ constexpr LaneRows make_lane_rows()
+{
+    constexpr PartialBlock<kBlock> t = make_partial_block<kBlock>();
+    constexpr PartialBlock<1> m = make_partial_block<1>();
+    static_assert(kBlock == 4, "three inner rows, 15 inputs");
+    LaneRows l{};
+    for (int c = 0; c < 15; c++) {
+        for (int r = 0; r < 12; r++) l.block[r][c] = (u32)t.f[r][c];
+        for (int j = 0; j < 3; j++) l.block[12 + j][c] = (u32)t.v[j][c];
+    }
+    for (int r = 0; r < 16; r++)
+        for (int c = 0; c < 12; c++) l.mds[r][c] = (u32)m.f[r % 12][c];
+    return l;
+}
+
+static __constant__ const LaneRows kLaneRowsDev = make_lane_rows();
+static const LaneRows kLaneRowsHost = make_lane_rows();
+
+ZK_HD const LaneRows &lane_rows()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return kLaneRowsDev;
+#else
+    return kLaneRowsHost;
+#endif
+}
+
+// sum_i c[i] t[i] for i in [FIRST, 12) on top of (a, b), by 32-bit halves.
+template <int FIRST>
+ZK_HD void row_sum(const u32 *c, const u64 t[12], u64 &a, u64 &b)
+{
+#pragma unroll
+    for (int i = FIRST; i < 12; i++) {
+        a += (u64)c[i] * (u32)t[i];
+        b += (u64)c[i] * (u32)(t[i] >> 32);
+    }
+}
+
+ZK_HD void row_add(u32 c, u64 y, u64 &a, u64 &b)
+{
+    a += (u64)c * (u32)y;
+    b += (u64)c * (u32)(y >> 32);
 }
 
 // The same permutation with canonical arithmetic only (no rare cases): the
@@ -411,7 +464,10 @@ ZK_HD u32 sponge_rows(u32 rem)
 // zero-padded; otherwise the overwrite-mode sponge (a final short chunk leaves
 // the stale rate lanes in place), digest = state[0..4).  `chunk(idx, m, v)` sees
 // each chunk of input once, right after it is fetched: elements idx .. idx+m-1
-// in v[0..m) (the exact recompute of a rare case fetches again, unseen).
+// in v[0..m) (the exact recompute of a rare case fetches again, unseen).  Rare
+// cases are redone at once, one permutation: redoing the whole sponge at its
+// end kept one wave busy for another 17 permutations of a 135-element leaf,
+// 0.1 to 0.4 ms of a 5.7 ms launch of 2^20 leaves in every third one.
 template <typename Get, typename Chunk>
 ZK_HD void hash_one_chunks(Get get, u32 n, u64 out[4], Chunk chunk)
 {
@@ -424,24 +480,31 @@ ZK_HD void hash_one_chunks(Get get, u32 n, u64 out[4], Chunk chunk)
     u64 s[12];
 #pragma unroll
     for (int i = 0; i < 12; i++) s[i] = 0;
-    bool rare = false;
     for (u32 idx = 0; idx < n; idx += 8) {
         const u32 rem = n - idx;
 #pragma unroll
         for (u32 i = 0; i < 8; i++)
             if (i < rem) s[i] = get(idx + i);
         chunk(idx, rem < 8 ? rem : 8u, (const u64 *)s);
+        u64 cap[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) cap[i] = s[8 + i];
+        bool rare = false;
         poseidon_permute(s, rare, sponge_rows(rem));
-    }
-    if (rare) {  // some lane hit a rare relaxed case: redo the sponge exactly
+        if (rare) {
+            // This lane hit a rare relaxed case: redo the permutation exactly
+            // from its inputs, the chunk (fetched again) and the capacity; a
+            // short chunk leaves rate elements of the state before it in
+            // place, which are not kept, so there the sponge is redone.
+            const u32 from = rem < 8 ? 0 : idx;
 #pragma unroll
-        for (int i = 0; i < 12; i++) s[i] = 0;
-        for (u32 idx = 0; idx < n; idx += 8) {
-            const u32 rem = n - idx;
+            for (int i = 0; i < 12; i++) s[i] = from && i >= 8 ? cap[i - 8] : 0;
+            for (u32 k = from; k <= idx; k += 8) {
 #pragma unroll
-            for (u32 i = 0; i < 8; i++)
-                if (i < rem) s[i] = get(idx + i);
-            poseidon_permute_safe(s);
+                for (u32 i = 0; i < 8; i++)
+                    if (i < n - k) s[i] = get(k + i);
+                poseidon_permute_safe(s);
+            }
         }
     }
 #pragma unroll
