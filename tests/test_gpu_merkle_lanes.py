@@ -64,3 +64,17 @@ def test_rare_case_leaves(Z, n_leaves, leaf_size):
     Z.fill_digests_buf_linear_gpu_with_gpu_ptr(dd, dc, dl, nd, 4, n_leaves, leaf_size, 2)
     odg, ocp = O.merkle(leaves, n_leaves, leaf_size, 2)
     assert (host(dc) == ocp).all() and (host(dd, 4 * nd) == odg).all()
+
+
+@pytest.mark.parametrize("leaf_size", [3, 4, 16, 17, 18, 33, 34, 35])
+def test_keccak_leaf_sizes(Z, leaf_size):
+    """Keccak leaves whose last block holds no, one, and all but one of the
+    17 words beside the padding; two-leaf subtrees and one deeper forest."""
+    from gpu_util import dev, empty, host
+    for n, h in ((64, 5), (256, 2)):
+        leaves = O.random(n * leaf_size, 40 + leaf_size)
+        nd = 2 * (n - (1 << h))
+        dl, dd, dc = dev(leaves), empty(4 * nd), empty(4 << h)
+        Z.fill_digests_buf_linear_gpu_with_gpu_ptr(dd, dc, dl, nd, 1 << h, n, leaf_size, h, hash_type=1)
+        odg, ocp = O.merkle(leaves, n, leaf_size, h, hash_type=1)
+        assert (host(dc) == ocp).all() and (host(dd, 4 * nd) == odg).all()

@@ -50,17 +50,79 @@ __host__ __device__ constexpr KeccakTables make_keccak_tables()
     return t;
 }
 
-ZK_HD u64 rotl64(u64 v, int n) { return n ? (v << n) | (v >> (64 - n)) : v; }
+// v rotated left by a constant n < 64: two funnel shifts on the device, where
+// the shift-and-or form compiles to four instructions.
+ZK_HD u64 rotl64(u64 v, int n)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    u32 lo = (u32)v, hi = (u32)(v >> 32);
+    if (n & 32) {
+        const u32 t = lo;
+        lo = hi;
+        hi = t;
+    }
+    if (n & 31) {
+        const u32 h = __builtin_amdgcn_alignbit(hi, lo, 32 - (n & 31));
+        lo = __builtin_amdgcn_alignbit(lo, hi, 32 - (n & 31));
+        hi = h;
+    }
+    return ((u64)hi << 32) | lo;
+#else
+    return n ? (v << n) | (v >> (64 - n)) : v;
+#endif
+}
 
+// a ^ b ^ c and a ^ (~b & c) as one three-input instruction for each half
+// (truth tables over a = 0xF0, b = 0xCC, c = 0xAA).
+ZK_HD u64 xor3(u64 a, u64 b, u64 c)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const u32 lo = __builtin_amdgcn_bitop3_b32((u32)a, (u32)b, (u32)c, 0x96);
+    const u32 hi = __builtin_amdgcn_bitop3_b32((u32)(a >> 32), (u32)(b >> 32), (u32)(c >> 32), 0x96);
+    return ((u64)hi << 32) | lo;
+#else
+    return a ^ b ^ c;
+#endif
+}
+
+ZK_HD u64 chi(u64 a, u64 b, u64 c)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const u32 lo = __builtin_amdgcn_bitop3_b32((u32)a, (u32)b, (u32)c, 0xD2);
+    const u32 hi = __builtin_amdgcn_bitop3_b32((u32)(a >> 32), (u32)(b >> 32), (u32)(c >> 32), 0xD2);
+    return ((u64)hi << 32) | lo;
+#else
+    return a ^ (~b & c);
+#endif
+}
+
+static __constant__ const KeccakTables kKeccakDev = make_keccak_tables();
+static const KeccakTables kKeccakHost = make_keccak_tables();
+
+ZK_HD const u64 *keccak_round_constants()
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return kKeccakDev.rc;
+#else
+    return kKeccakHost.rc;
+#endif
+}
+
+// Bound by instruction issue.  The rounds are a loop: unrolled, they are 34 KB
+// of instructions, and a leaf kernel with two copies outgrew the 64 KB
+// instruction cache.  190 vector instructions a round, 288 without the
+// three-input logic and the funnel shifts.  2^17 leaves of 85 elements: 194 us
+// unrolled, 171 as a loop, 120 with 190 instructions; a level 13 -> 11 us.
 ZK_HD void keccak_f1600(u64 A[25])
 {
     constexpr KeccakTables T = make_keccak_tables();
-    static_for<0, 24>([&](auto rc) {
-        constexpr int ir = decltype(rc)::value;
+    const u64 *rc = keccak_round_constants();
+#pragma unroll 1
+    for (int ir = 0; ir < 24; ir++) {
         u64 C[5], B[25];
         static_for<0, 5>([&](auto xc) {
             constexpr int x = decltype(xc)::value;
-            C[x] = A[x] ^ A[x + 5] ^ A[x + 10] ^ A[x + 15] ^ A[x + 20];
+            C[x] = xor3(xor3(A[x], A[x + 5], A[x + 10]), A[x + 15], A[x + 20]);
         });
         static_for<0, 5>([&](auto xc) {
             constexpr int x = decltype(xc)::value;
@@ -74,10 +136,10 @@ ZK_HD void keccak_f1600(u64 A[25])
         });
         static_for<0, 25>([&](auto ic) {
             constexpr int i = decltype(ic)::value, x = i % 5, y = i / 5;
-            A[i] = B[i] ^ (~B[(x + 1) % 5 + 5 * y] & B[(x + 2) % 5 + 5 * y]);
+            A[i] = chi(B[i], B[(x + 1) % 5 + 5 * y], B[(x + 2) % 5 + 5 * y]);
         });
-        A[0] ^= T.rc[ir];
-    });
+        A[0] ^= rc[ir];
+    }
 }
 
 // Plonky2's Keccak hasher as zeknox defines it (native/keccak/keccak.cu:
@@ -97,20 +159,17 @@ struct KeccakHasher {
         u64 A[25];
 #pragma unroll
         for (int i = 0; i < 25; i++) A[i] = 0;
-        u32 idx = 0;
-        for (; idx + 17 <= n; idx += 17) {
+        for (u32 idx = 0;; idx += 17) {
+            const u32 m = n - idx;  // words left; fewer than 17: the padding follows
+            u64 v[17];
 #pragma unroll
-            for (u32 w = 0; w < 17; w++) A[w] ^= get(idx + w);
+            for (u32 w = 0; w < 17; w++) v[w] = w < m ? get(idx + w) : (w == m ? 0x01 : 0);
+#pragma unroll
+            for (u32 w = 0; w < 17; w++) A[w] ^= v[w];
+            if (m < 17) A[16] ^= 0x8000000000000000ull;
             keccak_f1600(A);
+            if (m < 17) break;
         }
-        const u32 m = n - idx;  // 0 .. 16 words left, then the padding
-#pragma unroll
-        for (u32 w = 0; w < 17; w++) {
-            if (w < m) A[w] ^= get(idx + w);
-            if (w == m) A[w] ^= 0x01;
-        }
-        A[16] ^= 0x8000000000000000ull;
-        keccak_f1600(A);
         out[0] = A[0];
         out[1] = A[1];
         out[2] = A[2];
