@@ -21,6 +21,20 @@ static void expect(const char *what, u64 got, u128 want)
     if (gl_canon(got) != (u64)(want % ZK_P) && fails++ < 10) printf("%s: wrong value\n", what);
 }
 
+// sbox7_pair on the even and the odd lane of a pair, which must agree
+static u64 sbox_pair(u64 x, bool &rare)
+{
+    u64 y[2];
+    for (int odd = 0; odd < 2; odd++)
+        y[odd] = sbox7_pair(x, odd, [&](u64) {
+            u64 other = 0;  // what the other lane passes to its exchange
+            (void)sbox7_pair(x, !odd, [&](u64 r) { return other = r; }, rare);
+            return other;
+        }, rare);
+    if (y[0] != y[1] && fails++ < 10) printf("sbox7_pair: the lanes differ\n");
+    return y[0];
+}
+
 // poseidon_permute_hex_nc, lane by lane
 static void permute_hex(u64 st[12], bool &rare)
 {
@@ -51,7 +65,7 @@ static void permute_hex(u64 st[12], bool &rare)
     for (int blk = 0; blk < kBlocks; blk++) {
         const u64 *kp = rc + 12 * (kBlockStart + 1 + kBlock * blk);
         gather();
-        const u64 y0 = sbox7(t[0], rare);
+        const u64 y0 = sbox_pair(t[0], rare);
         for (u32 j = 0; j < 16; j++) {
             const u64 k = j >= 12 && j < 15 ? kp[12 * (j - 12)] : (j == 0 ? kp[36] : 0);
             a[j] = (u32)k;
@@ -62,7 +76,7 @@ static void permute_hex(u64 st[12], bool &rare)
         for (int q = 0; q < kBlock - 1; q++) {
             u64 v[16];
             for (u32 j = 0; j < 16; j++) v[j] = reduce_lohi64(a[j], b[j], rare);
-            const u64 y = sbox7(v[12 + q], rare);
+            const u64 y = sbox_pair(v[12 + q], rare);
             for (u32 j = 0; j < 16; j++) row_add(c[j].b[12 + q], y, a[j], b[j]);
         }
         for (u32 j = 0; j < 16; j++) s[j] = reduce_lohi64(a[j], b[j], rare);
@@ -100,7 +114,7 @@ static void permute_quad(u64 st[12], bool &rare)
         const u64 *kp = rc + 12 * (kBlockStart + 1 + kBlock * blk);
         u64 t[12], a[4][4], b[4][4];  // [lane][three rows, inner value]
         for (u32 e = 0; e < 12; e++) t[e] = s[e / 3][e % 3];
-        const u64 y0 = sbox7(t[0], rare);
+        const u64 y0 = sbox_pair(t[0], rare);
         for (u32 j = 0; j < 4; j++)
             for (int k = 0; k < 4; k++) {
                 const u32 *cc = k < 3 ? c[j].f[k] : c[j].v;
@@ -111,7 +125,7 @@ static void permute_quad(u64 st[12], bool &rare)
                 row_add(cc[0], y0, a[j][k], b[j][k]);
             }
         for (int q = 0; q < kBlock - 1; q++) {
-            const u64 y = sbox7(reduce_lohi64(a[q][3], b[q][3], rare), rare);
+            const u64 y = sbox_pair(reduce_lohi64(a[q][3], b[q][3], rare), rare);
             for (u32 j = 0; j < 4; j++) {
                 row_add(c[j].v[12 + q], y, a[j][3], b[j][3]);
                 for (int k = 0; k < 3; k++) row_add(c[j].f[k][12 + q], y, a[j][k], b[j][k]);

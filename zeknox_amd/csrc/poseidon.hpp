@@ -242,6 +242,31 @@ ZK_HD const u64 *folded_constants()
 #endif
 }
 
+// x^7 of a value that neighbouring lanes (l and l ^ 1) both hold, in three
+// products instead of four: the even lane forms x^2 x, the odd one x^2 x^2,
+// and both multiply their own by the other's (swap(r) is the neighbour's r).
+template <typename Swap>
+ZK_HD u64 sbox7_pair(u64 x, bool odd, Swap swap, bool &rare)
+{
+    const u64 x2 = gl_mul_nc<true>(x, x, rare);
+    const u64 r = gl_mul_nc<true>(x2, odd ? x2 : x, rare);
+    return gl_mul_nc<true>(r, swap(r), rare);
+}
+
+// The neighbouring lane's value (DPP quad_perm 1, 0, 3, 2).
+struct LaneSwap {
+    ZK_HD u64 operator()(u64 x) const
+    {
+#ifdef __HIP_DEVICE_COMPILE__
+        const u32 lo = (u32)__builtin_amdgcn_mov_dpp((int)(u32)x, 0xB1, 0xF, 0xF, false);
+        const u32 hi = (u32)__builtin_amdgcn_mov_dpp((int)(u32)(x >> 32), 0xB1, 0xF, 0xF, false);
+        return ((u64)hi << 32) | lo;
+#else
+        return x;  // device-only; a host emulation passes its own
+#endif
+    }
+};
+
 // A coefficient as a multiplier operand: small ones are instruction
 // immediates, the others scalar registers; powers of two are hidden from the
 // compiler (see mds_coeff).

@@ -10,8 +10,8 @@
 // for) and the lane's row of the layer, its coefficients in registers.  The
 // partial rounds go in blocks of four layers as in partial_block: lanes 0 .. 11
 // accumulate the rows of the block's result and lanes 12 .. 14, idle otherwise,
-// the three inner values of element 0 in the same instructions; every lane runs
-// the block's four S-boxes on the broadcast value.
+// the three inner values of element 0 in the same instructions; every lane pair
+// runs the block's four S-boxes on the broadcast value (sbox7_pair).
 //
 // The recomputation of a rare case (SAFE) runs round by round with the lanes'
 // elements exchanged by ds_bpermute, lanes 12 .. 15 holding copies.
@@ -141,11 +141,11 @@ ZK_DEV void poseidon_permute_hex_nc(u64 &s, u32 j, const HexCoefs &c, bool &rare
         u64 a = (u32)k, b = k >> 32;
         hex_gather(s, t);
         row_sum<1>(c.b, t, a, b);
-        u64 y = sbox7(t[0], rare);
+        u64 y = sbox7_pair(t[0], j & 1, LaneSwap(), rare);
         row_add(c.b[0], y, a, b);
         static_for<0, kBlock - 1>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            y = sbox7(hex_bcast<12 + q>(reduce_lohi64(a, b, rare)), rare);
+            y = sbox7_pair(hex_bcast<12 + q>(reduce_lohi64(a, b, rare)), j & 1, LaneSwap(), rare);
             row_add(c.b[12 + q], y, a, b);
         });
         s = reduce_lohi64(a, b, rare);

@@ -10,8 +10,8 @@
 // immediates.  The partial rounds go in blocks of four layers as in
 // partial_block: the state is broadcast once a block, each lane accumulates
 // its three rows of the block's result and, lanes 0 .. 2, one of the three
-// inner values of element 0 (coefficients in registers), and every lane runs
-// the block's four S-boxes.
+// inner values of element 0 (coefficients in registers), and every lane pair
+// runs the block's four S-boxes (sbox7_pair).
 //
 // The S-box and row phases are host-callable (a host emulation runs the four
 // lanes in lock step); only the gathers are device code.
@@ -180,7 +180,7 @@ ZK_DEV void poseidon_permute_quad_nc(u64 s[3], u32 j, const QuadCoefs &c, bool &
         }
         u64 av = (u32)kv, bv = kv >> 32, a[3] = {(u32)kf, 0, 0}, b[3] = {kf >> 32, 0, 0};
         row_sum<1>(c.v, t, av, bv);
-        u64 y = sbox7(t[0], rare);
+        u64 y = sbox7_pair(t[0], j & 1, LaneSwap(), rare);
         row_add(c.v[0], y, av, bv);
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -189,7 +189,7 @@ ZK_DEV void poseidon_permute_quad_nc(u64 s[3], u32 j, const QuadCoefs &c, bool &
         }
         static_for<0, kBlock - 1>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            y = sbox7(quad_bcast<q>(reduce_lohi64(av, bv, rare)), rare);
+            y = sbox7_pair(quad_bcast<q>(reduce_lohi64(av, bv, rare)), j & 1, LaneSwap(), rare);
             if constexpr (q < kBlock - 2) row_add(c.v[12 + q], y, av, bv);
 #pragma unroll
             for (int k = 0; k < 3; k++) row_add(c.f[k][12 + q], y, a[k], b[k]);
