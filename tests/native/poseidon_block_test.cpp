@@ -9,6 +9,7 @@
 #include <random>
 
 #include "../../zeknox_amd/csrc/poseidon_hex.hpp"
+#include "../../zeknox_amd/csrc/poseidon_mfma.hpp"
 #include "../../zeknox_amd/csrc/poseidon_quad.hpp"
 
 using namespace zk;
@@ -139,6 +140,52 @@ static void permute_quad(u64 st[12], bool &rare)
     for (u32 e = 0; e < 12; e++) st[e] = s[e / 3][e % 3];
 }
 
+// One layer as mds_mfma computes it for 64 lanes, with the MFMA's sums formed
+// here from its operand layout (A row m and B column m of lane m + 32 k are the
+// k half's 16 bytes; result register i of lane n + 32 g is row 8 (i / 4) + 4 g
+// + i % 4 of column n), against the layer by multiply-adds.
+static void check_mfma_layer(std::mt19937_64 &g)
+{
+    static const MfmaConsts mc = make_mfma_consts();
+    MfmaTiles t[64];
+    u64 s[64][12];
+    for (u32 l = 0; l < 64; l++) {
+        mfma_tiles(l, t[l]);
+        for (int i = 0; i < 12; i++) s[l][i] = l % 3 ? g() : (l & 1 ? ~0ull : 0);
+    }
+    auto byte = [](const v4i &v, int k) { return (int)(signed char)(v[k / 4] >> (8 * (k % 4))); };
+    const int round = (int)(g() % 3) + 1;
+    for (u32 l = 0; l < 64; l++) {
+        u64 want[12];
+        for (int i = 0; i < 12; i++) want[i] = s[l][i];
+        bool rare = false;
+        mds_fold(want, folded_constants() + 12 * round, kAllRows, rare);
+        for (int r = 0; r < 3; r++) {
+            int d[2][16] = {};
+            for (int half = 0; half < 2; half++)
+                for (int q = 0; q < 3; q++)
+                    for (int i = 0; i < 16; i++) {
+                        const u32 m = 8 * (i / 4) + 4 * (l >> 5) + i % 4;
+                        for (u32 kh = 0; kh < 2; kh++) {  // both k halves of column l % 32
+                            const u32 bl = (l & 31) + 32 * kh;
+                            v4i b;
+                            for (int j = 0; j < 4; j++) b[j] = (int)((u32)(s[bl][4 * q + j] >> (32 * half)) ^ 0x80808080u);
+                            const v4i &a = t[m + 32 * kh].w[r == 0 && q == 0 ? 3 : (q + 3 - r) % 3];
+                            for (int k = 0; k < 16; k++) d[half][i] += byte(a, k) * byte(b, k);
+                        }
+                    }
+            for (int e = 0; e < 4; e++) {
+                const u64 *k = mc.k[12 * round + 4 * r + e];
+                const u64 a = mfma_half(d[0][4 * e], d[0][4 * e + 1], d[0][4 * e + 2], d[0][4 * e + 3], k[0], 65536, 1);
+                const u64 b = mfma_half(d[1][4 * e], d[1][4 * e + 1], d[1][4 * e + 2], d[1][4 * e + 3], k[1], 65536, 1);
+                const u64 got = reduce_lohi42_nc(a, b, rare);
+                if (!rare && gl_canon(got) != gl_canon(want[4 * r + e]) && fails++ < 10)
+                    printf("mfma layer: lane %u row %d differs\n", l, 4 * r + e);
+            }
+        }
+    }
+}
+
 template <int K>
 static void row_sums()
 {
@@ -201,6 +248,7 @@ int main(int argc, char **argv)
         const u64 q = reduce_lohi42_nc(c, d, rare);
         if (!rare) expect("reduce_lohi42_nc", q, (u128)c + ((u128)d << 32));
     }
+    for (int it = 0; it < 6; it++) check_mfma_layer(g);
     row_sums<kBlock0>();
     row_sums<kBlock>();
     if (fails) return 1;

@@ -20,6 +20,7 @@
 #include "merkle.hpp"
 #include "poseidon.hpp"
 #include "poseidon_hex.hpp"
+#include "poseidon_mfma.hpp"
 #include "poseidon_quad.hpp"
 
 namespace zk {
@@ -66,18 +67,21 @@ TreeShape tree_shape(u64 n_digests, u64 n_caps, u64 n_leaves, u64 leaf_size, u64
     return t;
 }
 
-// The work of leaf thread t (one sponge per lane).  ring: the workgroup's
+// The work of leaf thread t (one sponge per lane; all lanes of a wave, those
+// past the last leaf hash leaf 0 and store nothing).  ring: the workgroup's
 // LDS ring of the row writer (ROWS only).
 template <LeafLayout LAYOUT, bool ROWS>
 __device__ __forceinline__ void leaf_hash_thread(const LeafArgs &a, u64 t, u64 *ring)
 {
-    if (t >= a.n_leaves) return;
+    const MfmaPermute perm;
+    const bool ok = t < a.n_leaves;
+    if (!ok) t = 0;
     u64 leaf;
     u64 h[4];
     if constexpr (LAYOUT == LeafLayout::RowMajor) {
         leaf = t;
         const u64 *p = a.leaves + leaf * a.leaf_size;
-        hash_one([p](u32 i) { return p[i]; }, a.leaf_size, h);
+        hash_one([p](u32 i) { return p[i]; }, a.leaf_size, h, perm);
     } else {
         // lane t owns LDE row t, i.e. leaf rev(t); with a.rows it also writes
         // that row to the row-major leaf matrix (what compute_transpose_rev
@@ -89,12 +93,15 @@ __device__ __forceinline__ void leaf_hash_thread(const LeafArgs &a, u64 t, u64 *
         if constexpr (ROWS) {
             RowSectorWriter w(a.rows, leaf, a.leaf_size, ring + threadIdx.x * kRowRingPitch);
             hash_one_chunks([p, cs](u32 i) { return p[(u64)i * cs]; }, a.leaf_size, h,
-                            [&w](u32, u32 m, const u64 *v) { w.chunk(m, v); });
-            w.finish();
+                            [&w, ok](u32, u32 m, const u64 *v) {
+                                if (ok) w.chunk(m, v);
+                            }, perm);
+            if (ok) w.finish();
         } else {
-            hash_one([p, cs](u32 i) { return p[(u64)i * cs]; }, a.leaf_size, h);
+            hash_one([p, cs](u32 i) { return p[(u64)i * cs]; }, a.leaf_size, h, perm);
         }
     }
+    if (!ok) return;
     u64 slot = leaf;
     if (a.sub_leaves) {
         const u64 s = leaf / a.sub_leaves, i = leaf % a.sub_leaves;
@@ -105,10 +112,10 @@ __device__ __forceinline__ void leaf_hash_thread(const LeafArgs &a, u64 t, u64 *
     for (int k = 0; k < 4; k++) o[k] = h[k];
 }
 
-// Exactly four waves per SIMD (102 VGPRs would allow it, 92 to 98 five): a
-// power of two of leaves then runs in whole rounds.  2^20 leaves of 135
-// elements take 5.7 ms; where the compiler found registers for five waves, the
-// fourth round ran on a fifth of the slots and they took 6.4 ms.
+// Exactly four waves per SIMD (118 VGPRs): a power of two of leaves then runs
+// in whole rounds.  2^20 leaves of 135 elements take 5.6 ms (5.7 without the
+// matrix cores); a build whose registers fitted five waves ran its fourth
+// round on a fifth of the slots and took 6.4 ms instead of 5.7.
 template <LeafLayout LAYOUT, bool ROWS>
 __global__ __launch_bounds__(kTreeLeafThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void leaf_hash_kernel(
     LeafArgs a)
@@ -216,12 +223,15 @@ __global__ __launch_bounds__(kTreeNodeThreads) void leaf_hash_hex_kernel(LeafArg
     a.out[slot * 4 + j] = h;
 }
 
-// One level: 2^r nodes per subtree starting at `base`.
+// One level: 2^r nodes per subtree starting at `base`.  Lanes past the last
+// node hash node 0 again and store nothing, so every wave stays complete.
 __global__ __launch_bounds__(kTreeNodeThreads) void level_hash_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub, u64 D)
 {
+    const MfmaPermute perm;
     const u64 t = (u64)blockIdx.x * kTreeNodeThreads + threadIdx.x;
-    if (t >= nodes * n_sub) return;
-    const u64 s = t / nodes, node = base + t % nodes;
+    const bool ok = t < nodes * n_sub;
+    const u64 tc = ok ? t : 0;
+    const u64 s = tc / nodes, node = base + tc % nodes;
     u64 *sd = d + s * D * 4;
     u64 l[4], r[4], o[4];
 #pragma unroll
@@ -229,7 +239,8 @@ __global__ __launch_bounds__(kTreeNodeThreads) void level_hash_kernel(u64 *d, u6
         l[k] = sd[(2 * node + 2) * 4 + k];
         r[k] = sd[(2 * node + 3) * 4 + k];
     }
-    hash_two(l, r, o);
+    hash_two(l, r, o, perm);
+    if (!ok) return;
 #pragma unroll
     for (int k = 0; k < 4; k++) sd[node * 4 + k] = o[k];
 }
@@ -297,14 +308,15 @@ __global__ __launch_bounds__(kNodeThreads) void level_hash_forest_kernel(const F
     const u64 *ca = sd + n.c0 * 4, *cb = ca + 4;
     u64 *o = n.out < 0 ? J.caps + n.s * 4 : sd + (u64)n.out * 4;
     if constexpr (G == 1) {
-        if (!ok) return;
+        const MfmaPermute perm;
         u64 l[4], r[4], h[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             l[k] = ca[k];
             r[k] = cb[k];
         }
-        hash_two(l, r, h);
+        hash_two(l, r, h, perm);
+        if (!ok) return;
 #pragma unroll
         for (int k = 0; k < 4; k++) o[k] = h[k];
     } else if constexpr (G == 4) {

@@ -450,8 +450,15 @@ ZK_HD void poseidon_permute_safe(u64 s[12])
     }
 }
 
+// The relaxed permutation as the sponges take it: perm(state, rare, rows
+// wanted).  (MfmaPermute in poseidon_mfma.hpp is the other.)
+struct PlainPermute {
+    ZK_HD void operator()(u64 s[12], bool &rare, u32 need) const { poseidon_permute(s, rare, need); }
+};
+
 // Two-to-one compression: state = [a, b, 0, 0, 0, 0] -> permute -> state[0..4).
-ZK_HD void hash_two(const u64 a[4], const u64 b[4], u64 out[4])
+template <typename Perm = PlainPermute>
+ZK_HD void hash_two(const u64 a[4], const u64 b[4], u64 out[4], const Perm &perm = Perm())
 {
     u64 s[12];
 #pragma unroll
@@ -461,7 +468,7 @@ ZK_HD void hash_two(const u64 a[4], const u64 b[4], u64 out[4])
         s[8 + i] = 0;
     }
     bool rare = false;
-    poseidon_permute(s, rare, 1u);  // the digest is rows 0 .. 3
+    perm(s, rare, 1u);  // the digest is rows 0 .. 3
     if (rare) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -493,8 +500,8 @@ ZK_HD u32 sponge_rows(u32 rem)
 // cases are redone at once, one permutation: redoing the whole sponge at its
 // end kept one wave busy for another 17 permutations of a 135-element leaf,
 // 0.1 to 0.4 ms of a 5.7 ms launch of 2^20 leaves in every third one.
-template <typename Get, typename Chunk>
-ZK_HD void hash_one_chunks(Get get, u32 n, u64 out[4], Chunk chunk)
+template <typename Get, typename Chunk, typename Perm = PlainPermute>
+ZK_HD void hash_one_chunks(Get get, u32 n, u64 out[4], Chunk chunk, const Perm &perm = Perm())
 {
     if (n <= 4) {
 #pragma unroll
@@ -515,7 +522,7 @@ ZK_HD void hash_one_chunks(Get get, u32 n, u64 out[4], Chunk chunk)
 #pragma unroll
         for (int i = 0; i < 4; i++) cap[i] = s[8 + i];
         bool rare = false;
-        poseidon_permute(s, rare, sponge_rows(rem));
+        perm(s, rare, sponge_rows(rem));
         if (rare) {
             // This lane hit a rare relaxed case: redo the permutation exactly
             // from its inputs, the chunk (fetched again) and the capacity; a
@@ -536,10 +543,10 @@ ZK_HD void hash_one_chunks(Get get, u32 n, u64 out[4], Chunk chunk)
     for (int i = 0; i < 4; i++) out[i] = gl_canon(s[i]);
 }
 
-template <typename Get>
-ZK_HD void hash_one(Get get, u32 n, u64 out[4])
+template <typename Get, typename Perm = PlainPermute>
+ZK_HD void hash_one(Get get, u32 n, u64 out[4], const Perm &perm = Perm())
 {
-    hash_one_chunks(get, n, out, [](u32, u32, const u64 *) {});
+    hash_one_chunks(get, n, out, [](u32, u32, const u64 *) {}, perm);
 }
 
 }  // namespace zk
