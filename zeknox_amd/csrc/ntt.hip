@@ -161,24 +161,26 @@ __global__ __launch_bounds__(kThreads) void ntt_fast_kernel(PassArgs a)
     fast_phase<BA, BB, INV>(a, tile, 1, threadIdx.x, kThreads, lds);
 }
 
-template <bool INV>
-__global__ __launch_bounds__(kR10Threads, 4) void ntt_r10_kernel(PassArgs a)
+// The 16-element passes: 10 bits (XB = 2) and 9 bits (XB = 1).
+template <int XB, bool INV>
+__global__ __launch_bounds__(kR10Threads, 4) void ntt_r16_kernel(PassArgs a)
 {
+    using R = R16<XB>;
     extern __shared__ u64 lds[];
-    u32 *votes = reinterpret_cast<u32 *>(lds + kR10Groups * kR10GP);
+    u32 *votes = reinterpret_cast<u32 *>(lds + R::G * R::GP);
     const u64 tile = a.tile_base + xcd_tile(blockIdx.x, gridDim.x);
     u32 col;
     u64 jhi, fast0;
-    Pass<10>::tile_decode(a, tile, col, jhi, fast0);
-    const bool last = (a.S + 10) == a.L;
+    Pass<R::B>::tile_decode(a, tile, col, jhi, fast0);
+    const bool last = (a.S + R::B) == a.L;
     const u32 tid = threadIdx.x;
     u64 out[16];
     bool rare = (a.flags & F_FORCE_EXACT) != 0;
-    r10_step_a<INV, false>(a, col, jhi, fast0, tid, lds, rare);
+    r16_step_a<XB, INV, false>(a, col, jhi, fast0, tid, lds, rare);
     __syncthreads();
-    r10_step_b<INV, false>(a, tid, lds, rare);
+    r16_step_b<XB, INV, false>(a, tid, lds, rare);
     __syncthreads();
-    r10_step_c<INV, false>(a, tid, lds, last, out, rare);
+    r16_step_c<XB, INV, false>(a, tid, lds, last, out, rare);
     // one vote per tile: each wave writes whether any of its lanes met a rare case
     const bool wave_rare = __builtin_amdgcn_ballot_w64(rare) != 0;
     if ((tid & 63) == 0) votes[tid >> 6] = wave_rare;
@@ -187,13 +189,13 @@ __global__ __launch_bounds__(kR10Threads, 4) void ntt_r10_kernel(PassArgs a)
 #pragma unroll
     for (u32 w = 0; w < kR10Threads / 64; w++) redo |= votes[w] != 0;
     if (redo) {
-        r10_step_a<INV, true>(a, col, jhi, fast0, tid, lds, rare);
+        r16_step_a<XB, INV, true>(a, col, jhi, fast0, tid, lds, rare);
         __syncthreads();
-        r10_step_b<INV, true>(a, tid, lds, rare);
+        r16_step_b<XB, INV, true>(a, tid, lds, rare);
         __syncthreads();
-        r10_step_c<INV, true>(a, tid, lds, last, out, rare);
+        r16_step_c<XB, INV, true>(a, tid, lds, last, out, rare);
     }
-    r10_store(a, col, jhi, fast0, tid, last, out);
+    r16_store<XB>(a, col, jhi, fast0, tid, last, out);
 }
 
 // Launches `kernel` over tiles [0, ntiles) in chunks whose grids stay below
@@ -210,17 +212,21 @@ static void launch_tiles(K kernel, PassArgs a, u64 ntiles, u32 threads, size_t l
     }
 }
 
-template <bool INV>
-static void launch_r10(const PassArgs &a, u64 ntiles, hipStream_t st)
+template <int XB, bool INV>
+static void launch_r16(const PassArgs &a, u64 ntiles, hipStream_t st)
 {
-    ZK_HIP(hipFuncSetAttribute((const void *)ntt_r10_kernel<INV>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)kR10Lds));
-    launch_tiles(ntt_r10_kernel<INV>, a, ntiles, kR10Threads, kR10Lds, st);
+    constexpr size_t lds = XB == 2 ? kR10Lds : kR9Lds;
+    ZK_HIP(hipFuncSetAttribute((const void *)ntt_r16_kernel<XB, INV>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds));
+    launch_tiles(ntt_r16_kernel<XB, INV>, a, ntiles, kR10Threads, lds, st);
 }
 
-static void launch_f10(const PassPlan &pp, bool inv, hipStream_t st)
+static void launch_f16(const PassPlan &pp, bool inv, hipStream_t st)
 {
-    inv ? launch_r10<true>(pp.a, pp.ntiles, st) : launch_r10<false>(pp.a, pp.ntiles, st);
+    if (pp.r10)
+        inv ? launch_r16<2, true>(pp.a, pp.ntiles, st) : launch_r16<2, false>(pp.a, pp.ntiles, st);
+    else
+        inv ? launch_r16<1, true>(pp.a, pp.ntiles, st) : launch_r16<1, false>(pp.a, pp.ntiles, st);
 }
 
 template <int B, bool INV>
@@ -439,8 +445,8 @@ void ntt_launch(DeviceCtx &c, const NttJob &job, hipStream_t st)
     for (size_t p = 0; p < passes.size(); p++) {
         const PassPlan &pp = passes[p];
         ProfScope ps(pass_name(job.prof_tag, (int)p), st);
-        if (pp.r10)
-            launch_f10(pp, job.inverse, st);
+        if (pp.r10 || pp.r9)
+            launch_f16(pp, job.inverse, st);
         else if (pp.fast)
             dispatch_fast(pp.B, job.inverse, pp.a, pp.ntiles, st);
         else

@@ -51,6 +51,7 @@ struct PassPlan {
     u64 ntiles;
     bool fast;
     bool r10;  // runs the 16-element 10-bit kernel (ntt_r10_kernel)
+    bool r9;   // or its 9-bit form
 };
 
 // Tuned plan of the transforms of one size 2^lg (lg <= 30), chosen by the
@@ -584,15 +585,36 @@ constexpr u32 kR10GP = 16 * kR10KP + 2;
 constexpr u32 kR10Groups = 8;
 constexpr u32 kR10Threads = 512;
 constexpr size_t kR10Lds = ((size_t)kR10Groups * kR10GP + kR10Threads / 64) * sizeof(u64);
+//
+// The 9-bit form (XB = 1; the passes of 2^17 .. 2^19-point transforms) is the
+// same with u < 2: J = t + 16 u + 32 v, k = kA + 16 kB + 32 kC, w32^(u kA) after
+// step A, 2-point DITs over u and w512^(rv (kA + 16 kB)) = every second entry
+// of the same table.  A group has 32 threads, a workgroup 16 groups (LDS pitch
+// 1 mod 16: the 16 lanes of an access are 16 groups).  In a first pass, where
+// a group's outputs are contiguous, step C takes kA fastest across lanes: the
+// stores are runs of 128 bytes instead of 32.
+template <int XB>
+struct R16 {
+    static constexpr int B = 8 + XB;         // bits of the pass
+    static constexpr u32 NX = 1u << XB;      // values of u
+    static constexpr u32 GB = 5 - XB;        // groups per workgroup (log2)
+    static constexpr u32 G = 1u << GB;
+    static constexpr u32 VS = 16 * NX;       // stride of v in J, of kC in k
+    static constexpr u32 KP = VS + 1;        // LDS pitch of kA
+    static constexpr u32 GP = 16 * KP + (XB == 2 ? 2 : 1);  // and of a group
+    static constexpr u32 TS = 64 / VS;       // stride in the w1024 table
+};
+static_assert(R16<2>::KP == kR10KP && R16<2>::GP == kR10GP && R16<2>::G == kR10Groups, "10-bit layout");
+constexpr size_t kR9Lds = ((size_t)R16<1>::G * R16<1>::GP + kR10Threads / 64) * sizeof(u64);
 
-// w64^(ru kA) of step A for the wave's ru, kA = 1..15 (constant exponents
-// per ru branch).
-template <int RU, bool INV, bool SAFE>
-ZK_HD void r10_w64(u64 v[16], bool &rare)
+// w_(16 NX)^(ru kA) of step A for the wave's ru, kA = 1..15 (constant
+// exponents per ru branch).
+template <int XB, int RU, bool INV, bool SAFE>
+ZK_HD void r16_twiddle_a(u64 v[16], bool &rare)
 {
     static_for<1, 16>([&](auto kc) {
         constexpr int kA = decltype(kc)::value;
-        constexpr int E = (root_exp2(6, INV) * RU * kA) % 192;
+        constexpr int E = (root_exp2(4 + XB, INV) * RU * kA) % 192;
         v[kA] = f_mul_root2<E, SAFE>(v[kA], rare);
     });
 }
@@ -601,15 +623,15 @@ ZK_HD void r10_w64(u64 v[16], bool &rare)
 // (the LDE's replication stages) or past the input; the others are loaded
 // with no lane-dependent branch (a lane past the input reads a.src[0], always
 // present, and keeps 0), so all of them are in flight together.
-template <int SKIP, bool SAFE>
-ZK_HD void r10_load_first(const PassArgs &a, const u64 *src, u64 n0, u64 lim, bool colok, u64 v[16])
+template <int XB, int SKIP, bool SAFE>
+ZK_HD void r16_load_first(const PassArgs &a, const u64 *src, u64 n0, u64 lim, bool colok, u64 v[16])
 {
     static_for<0, 16>([&](auto tc) {
         constexpr int t = decltype(tc)::value;
         if constexpr ((t & ((1 << SKIP) - 1)) != 0) {
             v[t] = 0;
         } else {
-            const u64 dn = (u64)(64 * ct_bitrev(t, 4)) << a.Jbits;
+            const u64 dn = (u64)(R16<XB>::VS * ct_bitrev(t, 4)) << a.Jbits;
             const bool ok = colok && n0 + dn < lim;
             const u64 x = *(ok ? src + dn : a.src);
             v[t] = ok ? (SAFE ? gl_canon(x) : x) : 0;
@@ -619,18 +641,20 @@ ZK_HD void r10_load_first(const PassArgs &a, const u64 *src, u64 n0, u64 lim, bo
 
 // Step A of thread tid: load 16 elements of one group, inter-pass twiddle or
 // coset factor, 16-point DIT, w64 twiddle, into LDS.
-template <bool INV, bool SAFE>
-ZK_HD void r10_step_a(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, u64 *lds, bool &rare)
+template <int XB, bool INV, bool SAFE>
+ZK_HD void r16_step_a(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, u64 *lds, bool &rare)
 {
-    const u32 g = tid & 7, v_ = (tid >> 3) & 15, u = tid >> 7;
-    const u32 J0 = 16 * u + 64 * v_;
+    using R = R16<XB>;
+    constexpr int B = R::B;
+    const u32 g = tid & (R::G - 1), v_ = (tid >> R::GB) & 15, u = tid >> (R::GB + 4);
+    const u32 J0 = 16 * u + R::VS * v_;
     u64 v[16];
     if (a.S > 0) {
         const u64 b = fast0 + g;
-        const u64 Jhi = jhi << 10;
+        const u64 Jhi = jhi << B;
         // per-thread base pointers, per-element offsets uniform across the
-        // workgroup (rev10(J0 + t) = rev10(J0) + 64 rev4(t))
-        if (a.flags & F_BLOCK_IN) {
+        // workgroup (rev_B(J0 + t) = rev_B(J0) + VS rev4(t))
+        if (XB == 2 && (a.flags & F_BLOCK_IN)) {
             // blocked intermediate (Jbits = 0): element (b, J) at
             // (b >> 3) 2^(B+3) + rev_B(J) 8 + (b & 7)
             const u64 *src = a.src + (u64)col * a.src_stride + ((b >> 3) << 13) + (b & 7) +
@@ -666,7 +690,7 @@ ZK_HD void r10_step_a(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, u
             const u32 jb = a.L - a.S;
             const u64 mask = (1ull << a.L) - 1;
             const u64 ub = (bp << a.Sprev) & mask;
-            const u64 rhi = zk_bitrev((u32)((J0 >> 4) + (jhi << 6)), jb - 4);
+            const u64 rhi = zk_bitrev((u32)((J0 >> 4) + (jhi << (B - 4))), jb - 4);
             const u64 base = root_pow(a.pw, a.L, (ub * rhi) & mask);
             const u64 step = root_pow(a.pw, a.L, (ub << (jb - 4)) & mask);
             const u64 step2 = f_mul<SAFE>(step, step, rare);
@@ -684,25 +708,25 @@ ZK_HD void r10_step_a(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, u
         }
     } else {
         // first pass of a multi-pass transform: element J is natural index
-        // n = rev10(J) 2^Jbits + (the group's fast index)
+        // n = rev_B(J) 2^Jbits + (the group's fast index)
         const u64 nlow = fast0 + g;
-        const u64 n0 = ((u64)zk_bitrev(J0, 10) << a.Jbits) + nlow;  // + (64 rev4(t) << Jbits)
+        const u64 n0 = ((u64)zk_bitrev(J0, B) << a.Jbits) + nlow;  // + (VS rev4(t) << Jbits)
         const u64 *src = a.src + (u64)col * a.src_stride + n0;
         const u64 lim = 1ull << a.lg_in;
         const u32 skipmask = (1u << a.skip) - 1;
         const bool colok = col < a.ncols;
         switch (a.skip) {  // uniform
-        case 0: r10_load_first<0, SAFE>(a, src, n0, lim, colok, v); break;
-        case 1: r10_load_first<1, SAFE>(a, src, n0, lim, colok, v); break;
-        case 2: r10_load_first<2, SAFE>(a, src, n0, lim, colok, v); break;
-        case 3: r10_load_first<3, SAFE>(a, src, n0, lim, colok, v); break;
-        default: r10_load_first<4, SAFE>(a, src, n0, lim, colok, v); break;
+        case 0: r16_load_first<XB, 0, SAFE>(a, src, n0, lim, colok, v); break;
+        case 1: r16_load_first<XB, 1, SAFE>(a, src, n0, lim, colok, v); break;
+        case 2: r16_load_first<XB, 2, SAFE>(a, src, n0, lim, colok, v); break;
+        case 3: r16_load_first<XB, 3, SAFE>(a, src, n0, lim, colok, v); break;
+        default: r16_load_first<XB, 4, SAFE>(a, src, n0, lim, colok, v); break;
         }
         if (a.flags & F_COSET_IN) {
 #pragma unroll
             for (int t = 0; t < 16; t++) {
                 if (t & skipmask) continue;
-                const u64 n = ((u64)zk_bitrev(J0 + t, 10) << a.Jbits) + nlow;
+                const u64 n = ((u64)zk_bitrev(J0 + t, B) << a.Jbits) + nlow;
                 const u64 c0 = a.gpw[n & (kPowLen - 1)];
                 const u64 c1 = a.gpw[kPowLen + ((n >> kPowBits) & (kPowLen - 1))];
                 const u64 c2 = a.gpw[2 * kPowLen + (n >> (2 * kPowBits))];
@@ -711,43 +735,68 @@ ZK_HD void r10_step_a(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, u
         }
     }
     dit_pow2<4, INV, SAFE>(v, a.S > 0 ? 0 : (int)a.skip, rare);
-    switch (zk_bitrev(u, 2)) {  // uniform across the wave
-    case 1: r10_w64<1, INV, SAFE>(v, rare); break;
-    case 2: r10_w64<2, INV, SAFE>(v, rare); break;
-    case 3: r10_w64<3, INV, SAFE>(v, rare); break;
+    switch (zk_bitrev(u, XB)) {  // uniform across the wave
+    case 1: r16_twiddle_a<XB, 1, INV, SAFE>(v, rare); break;
+    case 2:
+        if constexpr (XB == 2) r16_twiddle_a<XB, 2, INV, SAFE>(v, rare);
+        break;
+    case 3:
+        if constexpr (XB == 2) r16_twiddle_a<XB, 3, INV, SAFE>(v, rare);
+        break;
     default: break;
     }
-    u64 *row = lds + g * kR10GP + 16 * u + v_;
+    u64 *row = lds + g * R::GP + 16 * u + v_;
 #pragma unroll
-    for (int kA = 0; kA < 16; kA++) row[kA * kR10KP] = v[kA];
+    for (int kA = 0; kA < 16; kA++) row[kA * R::KP] = v[kA];
 }
 
-// Step B of thread tid: four 4-point DITs over u (kA = 4 (tid >> 7) + i),
-// w1024 twiddle, in place (each thread rewrites exactly the 16 entries it read).
-template <bool INV, bool SAFE>
-ZK_HD void r10_step_b(const PassArgs &a, u32 tid, u64 *lds, bool &rare)
+// Step B of thread tid: 16 / NX NX-point DITs over u (kA = (16 / NX) w + i),
+// w1024 (w512) twiddle, in place (each thread rewrites exactly the 16 entries
+// it read).
+template <int XB, bool INV, bool SAFE>
+ZK_HD void r16_step_b(const PassArgs &a, u32 tid, u64 *lds, bool &rare)
 {
-    const u32 g = tid & 7, v_ = (tid >> 3) & 15, kAh = tid >> 7;
-    u64 *base = lds + g * kR10GP + (4 * kAh) * kR10KP + v_;
-    const u64 *tb = a.tb + 64 * v_ + 4 * kAh;  // w1024^(rv j), j = kA + 16 kB
+    using R = R16<XB>;
+    constexpr u32 NI = 16 / R::NX;
+    const u32 g = tid & (R::G - 1), v_ = (tid >> R::GB) & 15, kAh = tid >> (R::GB + 4);
+    u64 *base = lds + g * R::GP + (NI * kAh) * R::KP + v_;
+    const u64 *tb = a.tb + 64 * v_ + R::TS * NI * kAh;  // w1024^(rv j TS), j = kA + 16 kB
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        u64 y[4];
+    for (u32 i = 0; i < NI; i++) {
+        u64 y[R::NX];
 #pragma unroll
-        for (int x = 0; x < 4; x++) y[x] = SAFE ? gl_canon(base[i * kR10KP + 16 * x]) : base[i * kR10KP + 16 * x];
-        dit_pow2<2, INV, SAFE>(y, 0, rare);
+        for (u32 x = 0; x < R::NX; x++) y[x] = SAFE ? gl_canon(base[i * R::KP + 16 * x]) : base[i * R::KP + 16 * x];
+        dit_pow2<XB, INV, SAFE>(y, 0, rare);
 #pragma unroll
-        for (int kB = 0; kB < 4; kB++) base[i * kR10KP + 16 * kB] = f_mul<SAFE>(y[kB], tb[i + 16 * kB], rare);
+        for (u32 kB = 0; kB < R::NX; kB++)
+            base[i * R::KP + 16 * kB] = f_mul<SAFE>(y[kB], tb[R::TS * (i + 16 * kB)], rare);
     }
 }
 
-// Step C of thread tid (kA = (tid >> 3) & 15, kB = tid >> 7): 16-point DIT
-// over v; out[kC] is output index kA + 16 kB + 64 kC.
-template <bool INV, bool SAFE>
-ZK_HD void r10_step_c(const PassArgs &a, u32 tid, const u64 *lds, bool last, u64 out[16], bool &rare)
+// Step C's role of thread tid: group g, outputs kA + 16 kB + VS kC.
+template <int XB>
+ZK_HD void r16_role_c(const PassArgs &a, u32 tid, u32 &g, u32 &kA, u32 &kB)
 {
-    const u32 g = tid & 7, kA = (tid >> 3) & 15, kB = tid >> 7;
-    const u64 *row = lds + g * kR10GP + kA * kR10KP + 16 * kB;
+    using R = R16<XB>;
+    g = tid & (R::G - 1);
+    kA = (tid >> R::GB) & 15;
+    kB = tid >> (R::GB + 4);
+    if (XB == 1 && a.S == 0) {
+        const u32 x = g;
+        g = kA;
+        kA = x;
+    }
+}
+
+// Step C of thread tid: 16-point DIT over v; out[kC] is output index kA + 16 kB
+// + VS kC.
+template <int XB, bool INV, bool SAFE>
+ZK_HD void r16_step_c(const PassArgs &a, u32 tid, const u64 *lds, bool last, u64 out[16], bool &rare)
+{
+    using R = R16<XB>;
+    u32 g, kA, kB;
+    r16_role_c<XB>(a, tid, g, kA, kB);
+    const u64 *row = lds + g * R::GP + kA * R::KP + 16 * kB;
 #pragma unroll
     for (int v = 0; v < 16; v++) out[v] = SAFE ? gl_canon(row[v]) : row[v];
     dit_pow2<4, INV, SAFE>(out, 0, rare);
@@ -757,23 +806,27 @@ ZK_HD void r10_step_c(const PassArgs &a, u32 tid, const u64 *lds, bool last, u64
     }
 }
 
-ZK_HD void r10_store(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, bool last, const u64 out[16])
+template <int XB>
+ZK_HD void r16_store(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, bool last, const u64 out[16])
 {
-    const u32 g = tid & 7, kA = (tid >> 3) & 15, kB = tid >> 7;
+    using R = R16<XB>;
+    constexpr int B = R::B;
+    u32 g, kA, kB;
+    r16_role_c<XB>(a, tid, g, kA, kB);
     if (col >= a.ncols) return;
-    // output index k = k0 + 64 kC; position = pos0 + (uniform offset)
+    // output index k = k0 + VS kC; position = pos0 + (uniform offset)
     const u64 k0 = kA + 16 * kB;
     u64 pos0;
     u32 sh;
     if (a.S > 0) {
-        pos0 = fast0 + g + ((k0 + (jhi << 10)) << a.S);
-        sh = a.S + 6;
-    } else if (a.flags & F_BLOCK_OUT) {  // blocked for the next pass (its b = k, rev(J) = f)
+        pos0 = fast0 + g + ((k0 + (jhi << B)) << a.S);
+        sh = a.S + 4 + XB;
+    } else if (XB == 2 && (a.flags & F_BLOCK_OUT)) {  // blocked for the next pass (its b = k, rev(J) = f)
         pos0 = ((k0 >> 3) << (a.Jbits + 3)) + ((fast0 + g) << 3) + (k0 & 7);
         sh = a.Jbits + 6;  // 64 kC >> 3 = 8 kC blocks of 2^(Jbits+3)
     } else {
-        pos0 = k0 + ((u64)zk_bitrev((u32)(fast0 + g), a.Jbits) << 10);
-        sh = 6;
+        pos0 = k0 + ((u64)zk_bitrev((u32)(fast0 + g), a.Jbits) << B);
+        sh = 4 + XB;
     }
     u64 *dst = a.dst + (u64)col * a.dst_stride + pos0;
 #pragma unroll
@@ -789,9 +842,36 @@ ZK_HD void r10_store(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, bo
     }
 }
 
+// The 10-bit pass by its own names.
+template <bool INV, bool SAFE>
+ZK_HD void r10_step_a(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, u64 *lds, bool &rare)
+{
+    r16_step_a<2, INV, SAFE>(a, col, jhi, fast0, tid, lds, rare);
+}
+
+template <bool INV, bool SAFE>
+ZK_HD void r10_step_b(const PassArgs &a, u32 tid, u64 *lds, bool &rare)
+{
+    r16_step_b<2, INV, SAFE>(a, tid, lds, rare);
+}
+
+template <bool INV, bool SAFE>
+ZK_HD void r10_step_c(const PassArgs &a, u32 tid, const u64 *lds, bool last, u64 out[16], bool &rare)
+{
+    r16_step_c<2, INV, SAFE>(a, tid, lds, last, out, rare);
+}
+
+ZK_HD void r10_store(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, bool last, const u64 out[16])
+{
+    r16_store<2>(a, col, jhi, fast0, tid, last, out);
+}
+
 // Groups per workgroup of the 16-element pass (log2): 8 groups, two
 // workgroups per CU.
 inline u32 f10_gbits(const PassArgs &) { return 3; }
+
+// Groups per workgroup of the 9-bit form (log2).
+constexpr u32 kR9Gbits = R16<1>::GB;
 
 // The 16-element pass applies to 10-bit passes whose workgroup holds the
 // groups of one column: passes after the first, and first passes of
@@ -803,11 +883,18 @@ inline bool use_fast10(u32 B, const PassArgs &a)
     return B == 10 && extent >= (1ull << f10_gbits(a));
 }
 
+// Likewise the 9-bit form, for 9-bit passes whose fast dimension has its 16
+// groups.
+inline bool use_fast9(u32 B, const PassArgs &a)
+{
+    return B == 9 && (a.S > 0 ? a.S : a.Jbits) >= kR9Gbits;
+}
+
 // Re-tiles a pass for the 16-element kernel: its groups per workgroup.
-inline void f10_retile(PassPlan &pp)
+inline void f16_retile(PassPlan &pp, u32 gbits)
 {
     PassArgs &a = pp.a;
-    a.Gbits = f10_gbits(a);
+    a.Gbits = gbits;
     if (a.S > 0)
         pp.ntiles = (u64)a.ncols * (1ull << a.Jbits) * ((1ull << a.S) >> a.Gbits);
     else
@@ -949,9 +1036,11 @@ inline std::vector<PassPlan> plan_passes(const NttJob &job, const u64 *pw, const
         // first pass of a zero-extended input: the first L - lg_in DIT stages
         // of every step-A block only replicate
         a.skip = (S == 0 && fast) ? std::min<u32>(job.lg - job.lg_in, (B + 1) / 2) : 0;
-        PassPlan pp{a, B, ntiles, fast, false};
+        PassPlan pp{a, B, ntiles, fast, false, false};
         pp.r10 = fast && (!tune.np || tune.r10[p]) && use_fast10(B, a);
-        if (pp.r10) f10_retile(pp);
+        if (pp.r10) f16_retile(pp, f10_gbits(a));
+        pp.r9 = fast && (!tune.np || tune.r10[p]) && use_fast9(B, a);
+        if (pp.r9) f16_retile(pp, kR9Gbits);
         out.push_back(pp);
         Sprev = S;
         S += B;
