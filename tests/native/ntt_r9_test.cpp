@@ -1,4 +1,4 @@
-// The 9-bit form of the 16-element pass (r16_*<1>), run thread by thread in
+// The 9-bit and 8-bit forms of the 16-element pass (r16_*<1>, <0>), run thread by thread in
 // kernel order, against the general pass (fast_phase) on the same plans: both
 // computations of each transform must agree bit for bit.  Usage: ntt_r9_test;
 // prints "ok, N transforms".
@@ -12,26 +12,28 @@
 
 using namespace zk;
 
-template <bool INV>
-static void run_r9(const PassArgs &a, u64 ntiles)
+template <int XB, bool INV>
+static void run_r16(const PassArgs &a, u64 ntiles)
 {
-    std::vector<u64> lds((size_t)R16<1>::G * R16<1>::GP);
+    std::vector<u64> lds((size_t)R16<XB>::G * R16<XB>::GP);
     std::vector<u64> out(16 * kR10Threads);
     for (u64 b = 0; b < ntiles; b++) {
         u32 col;
         u64 jhi, fast0;
-        Pass<9>::tile_decode(a, xcd_tile(b, ntiles), col, jhi, fast0);
-        const bool last = (a.S + 9) == a.L;
+        Pass<8 + XB>::tile_decode(a, xcd_tile(b, ntiles), col, jhi, fast0);
+        const bool last = (a.S + 8 + XB) == a.L;
         bool any = (a.flags & F_FORCE_EXACT) != 0;
-        for (u32 t = 0; t < kR10Threads; t++) r16_step_a<1, INV, false>(a, col, jhi, fast0, t, lds.data(), any);
-        for (u32 t = 0; t < kR10Threads; t++) r16_step_b<1, INV, false>(a, t, lds.data(), any);
-        for (u32 t = 0; t < kR10Threads; t++) r16_step_c<1, INV, false>(a, t, lds.data(), last, &out[16 * t], any);
+        for (u32 t = 0; t < kR10Threads; t++) r16_step_a<XB, INV, false>(a, col, jhi, fast0, t, lds.data(), any);
+        if constexpr (XB > 0)
+            for (u32 t = 0; t < kR10Threads; t++) r16_step_b<XB, INV, false>(a, t, lds.data(), any);
+        for (u32 t = 0; t < kR10Threads; t++) r16_step_c<XB, INV, false>(a, t, lds.data(), last, &out[16 * t], any);
         if (any) {
-            for (u32 t = 0; t < kR10Threads; t++) r16_step_a<1, INV, true>(a, col, jhi, fast0, t, lds.data(), any);
-            for (u32 t = 0; t < kR10Threads; t++) r16_step_b<1, INV, true>(a, t, lds.data(), any);
-            for (u32 t = 0; t < kR10Threads; t++) r16_step_c<1, INV, true>(a, t, lds.data(), last, &out[16 * t], any);
+            for (u32 t = 0; t < kR10Threads; t++) r16_step_a<XB, INV, true>(a, col, jhi, fast0, t, lds.data(), any);
+            if constexpr (XB > 0)
+                for (u32 t = 0; t < kR10Threads; t++) r16_step_b<XB, INV, true>(a, t, lds.data(), any);
+            for (u32 t = 0; t < kR10Threads; t++) r16_step_c<XB, INV, true>(a, t, lds.data(), last, &out[16 * t], any);
         }
-        for (u32 t = 0; t < kR10Threads; t++) r16_store<1>(a, col, jhi, fast0, t, last, &out[16 * t]);
+        for (u32 t = 0; t < kR10Threads; t++) r16_store<XB>(a, col, jhi, fast0, t, last, &out[16 * t]);
     }
 }
 
@@ -48,10 +50,12 @@ static void run_fast(const PassArgs &a, u64 ntiles)
 template <bool INV>
 static void run_pass(const PassPlan &pp)
 {
-    if (pp.r9) return run_r9<INV>(pp.a, pp.ntiles);
+    if (pp.r9) return run_r16<1, INV>(pp.a, pp.ntiles);
+    if (pp.r8) return run_r16<0, INV>(pp.a, pp.ntiles);
     switch (pp.B) {
     case 4: return run_fast<4, INV>(pp.a, pp.ntiles);
     case 5: return run_fast<5, INV>(pp.a, pp.ntiles);
+    case 8: return run_fast<8, INV>(pp.a, pp.ntiles);
     case 9: return run_fast<9, INV>(pp.a, pp.ntiles);
     default: printf("pass of %u bits not run here\n", pp.B);
     }
@@ -106,7 +110,7 @@ static std::vector<u64> transform(u32 lg, u32 lg_in, u32 ncols, bool inv, bool c
                 tws.back()[i] = twiddle_entry(pw[inv].data(), pp.a.L, pp.a.S, pp.a.Sprev, i);
             pp.a.tw = tws.back().data();
         }
-        nr9 += pp.r9;
+        nr9 += pp.r9 || pp.r8;
         inv ? run_pass<true>(pp) : run_pass<false>(pp);
     }
     ntt_tune_table()[lg] = NttTune{};
@@ -129,15 +133,16 @@ int main()
     }
     std::mt19937_64 g(9);
     int runs = 0, fails = 0, nr9 = 0;
-    // first, middle and last passes; 16 groups exactly (4-bit neighbour) and more
-    const std::vector<std::vector<u32>> plans = {{9, 4}, {4, 9}, {9, 5}, {5, 9}, {4, 9, 4}, {9, 9}};
+    // first, middle and last passes; 16 (32) groups exactly and more
+    const std::vector<std::vector<u32>> plans = {{9, 4}, {4, 9}, {9, 5}, {5, 9}, {4, 9, 4},
+                                                 {8, 5}, {8, 9}};
     for (const auto &bits : plans) {
         u32 lg = 0;
         for (u32 b : bits) lg += b;
         for (int inv = 0; inv < 2; inv++)
-            for (u32 r = 0; r < (inv ? 1u : 7u); r++)
+            for (u32 r = 0; r < (inv ? 1u : 7u); r += r < 3 ? 1 : 3)
                 for (int form = 0; form < 4; form++) {
-                    if (lg == 18 && (form == 1 || r > 1)) continue;  // the large plan: fewer forms
+                    if (lg >= 16 && (form == 1 || form == 2 || r > 1)) continue;  // the larger plans: fewer forms
                     const u32 ncols = form == 2 ? 3 : 1;
                     const bool coset = form != 1, force = form == 3, table = form < 2, place = form == 2;
                     std::vector<u64> in((size_t)ncols << (lg - r));
@@ -151,6 +156,6 @@ int main()
                 }
     }
     if (!nr9) fails++;
-    printf("%s, %d transforms, %d 9-bit passes\n", fails ? "FAIL" : "ok", runs, nr9);
+    printf("%s, %d transforms, %d 16-element passes\n", fails ? "FAIL" : "ok", runs, nr9);
     return fails ? 1 : 0;
 }

@@ -1,5 +1,5 @@
-"""The 9-bit form of the 16-element NTT pass (zeknox_amd/csrc/ntt_pass.hpp),
-its per-thread code run on the host under AddressSanitizer and UBSan, against
+"""The 9-bit and 8-bit forms of the 16-element NTT pass (zeknox_amd/csrc/ntt_pass.hpp),
+their per-thread code run on the host under AddressSanitizer and UBSan, against
 the general pass: as first, middle and last pass, forward, inverse and LDE (0
 to 6 skipped bits), with and without the coset, the twiddle table, a scratch
 buffer and the forced exact path."""
@@ -13,7 +13,7 @@ HIPCC = "/opt/rocm/bin/hipcc"
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
-def test_nine_bit_pass_equals_general_pass(tmp_path):
+def test_small_forms_equal_general_pass(tmp_path):
     exe = str(tmp_path / "ntt_r9_test")
     src = os.path.join(ROOT, "tests", "native", "ntt_r9_test.cpp")
     r = subprocess.run([HIPCC, "-x", "hip", "--cuda-host-only", "-O2", "-std=c++17", "-I" + os.path.join(ROOT, "include"),

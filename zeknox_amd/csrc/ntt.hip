@@ -161,7 +161,7 @@ __global__ __launch_bounds__(kThreads) void ntt_fast_kernel(PassArgs a)
     fast_phase<BA, BB, INV>(a, tile, 1, threadIdx.x, kThreads, lds);
 }
 
-// The 16-element passes: 10 bits (XB = 2) and 9 bits (XB = 1).
+// The 16-element passes: 10 bits (XB = 2), 9 bits (1) and 8 bits (0).
 template <int XB, bool INV>
 __global__ __launch_bounds__(kR10Threads, 4) void ntt_r16_kernel(PassArgs a)
 {
@@ -178,8 +178,10 @@ __global__ __launch_bounds__(kR10Threads, 4) void ntt_r16_kernel(PassArgs a)
     bool rare = (a.flags & F_FORCE_EXACT) != 0;
     r16_step_a<XB, INV, false>(a, col, jhi, fast0, tid, lds, rare);
     __syncthreads();
-    r16_step_b<XB, INV, false>(a, tid, lds, rare);
-    __syncthreads();
+    if constexpr (XB > 0) {
+        r16_step_b<XB, INV, false>(a, tid, lds, rare);
+        __syncthreads();
+    }
     r16_step_c<XB, INV, false>(a, tid, lds, last, out, rare);
     // one vote per tile: each wave writes whether any of its lanes met a rare case
     const bool wave_rare = __builtin_amdgcn_ballot_w64(rare) != 0;
@@ -191,8 +193,10 @@ __global__ __launch_bounds__(kR10Threads, 4) void ntt_r16_kernel(PassArgs a)
     if (redo) {
         r16_step_a<XB, INV, true>(a, col, jhi, fast0, tid, lds, rare);
         __syncthreads();
-        r16_step_b<XB, INV, true>(a, tid, lds, rare);
-        __syncthreads();
+        if constexpr (XB > 0) {
+            r16_step_b<XB, INV, true>(a, tid, lds, rare);
+            __syncthreads();
+        }
         r16_step_c<XB, INV, true>(a, tid, lds, last, out, rare);
     }
     r16_store<XB>(a, col, jhi, fast0, tid, last, out);
@@ -215,18 +219,26 @@ static void launch_tiles(K kernel, PassArgs a, u64 ntiles, u32 threads, size_t l
 template <int XB, bool INV>
 static void launch_r16(const PassArgs &a, u64 ntiles, hipStream_t st)
 {
-    constexpr size_t lds = XB == 2 ? kR10Lds : kR9Lds;
+    constexpr size_t lds = XB == 2 ? kR10Lds : (XB == 1 ? kR9Lds : kR8Lds);
     ZK_HIP(hipFuncSetAttribute((const void *)ntt_r16_kernel<XB, INV>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)lds));
     launch_tiles(ntt_r16_kernel<XB, INV>, a, ntiles, kR10Threads, lds, st);
 }
 
+template <int XB>
+static void launch_r16(const PassPlan &pp, bool inv, hipStream_t st)
+{
+    inv ? launch_r16<XB, true>(pp.a, pp.ntiles, st) : launch_r16<XB, false>(pp.a, pp.ntiles, st);
+}
+
 static void launch_f16(const PassPlan &pp, bool inv, hipStream_t st)
 {
     if (pp.r10)
-        inv ? launch_r16<2, true>(pp.a, pp.ntiles, st) : launch_r16<2, false>(pp.a, pp.ntiles, st);
+        launch_r16<2>(pp, inv, st);
+    else if (pp.r9)
+        launch_r16<1>(pp, inv, st);
     else
-        inv ? launch_r16<1, true>(pp.a, pp.ntiles, st) : launch_r16<1, false>(pp.a, pp.ntiles, st);
+        launch_r16<0>(pp, inv, st);
 }
 
 template <int B, bool INV>
@@ -445,7 +457,7 @@ void ntt_launch(DeviceCtx &c, const NttJob &job, hipStream_t st)
     for (size_t p = 0; p < passes.size(); p++) {
         const PassPlan &pp = passes[p];
         ProfScope ps(pass_name(job.prof_tag, (int)p), st);
-        if (pp.r10 || pp.r9)
+        if (pp.r10 || pp.r9 || pp.r8)
             launch_f16(pp, job.inverse, st);
         else if (pp.fast)
             dispatch_fast(pp.B, job.inverse, pp.a, pp.ntiles, st);

@@ -52,6 +52,7 @@ struct PassPlan {
     bool fast;
     bool r10;  // runs the 16-element 10-bit kernel (ntt_r10_kernel)
     bool r9;   // or its 9-bit form
+    bool r8;   // or its 8-bit form
 };
 
 // Tuned plan of the transforms of one size 2^lg (lg <= 30), chosen by the
@@ -593,6 +594,9 @@ constexpr size_t kR10Lds = ((size_t)kR10Groups * kR10GP + kR10Threads / 64) * si
 // 1 mod 16: the 16 lanes of an access are 16 groups).  In a first pass, where
 // a group's outputs are contiguous, step C takes kA fastest across lanes: the
 // stores are runs of 128 bytes instead of 32.
+//
+// The 8-bit form (XB = 0; first passes) has no u: step A ends with w256^(rv kA)
+// (every fourth entry of the table) and step B falls away; 32 groups.
 template <int XB>
 struct R16 {
     static constexpr int B = 8 + XB;         // bits of the pass
@@ -604,6 +608,7 @@ struct R16 {
     static constexpr u32 GP = 16 * KP + (XB == 2 ? 2 : 1);  // and of a group
     static constexpr u32 TS = 64 / VS;       // stride in the w1024 table
 };
+constexpr size_t kR8Lds = ((size_t)R16<0>::G * R16<0>::GP + kR10Threads / 64) * sizeof(u64);
 static_assert(R16<2>::KP == kR10KP && R16<2>::GP == kR10GP && R16<2>::G == kR10Groups, "10-bit layout");
 constexpr size_t kR9Lds = ((size_t)R16<1>::G * R16<1>::GP + kR10Threads / 64) * sizeof(u64);
 
@@ -736,7 +741,9 @@ ZK_HD void r16_step_a(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, u
     }
     dit_pow2<4, INV, SAFE>(v, a.S > 0 ? 0 : (int)a.skip, rare);
     switch (zk_bitrev(u, XB)) {  // uniform across the wave
-    case 1: r16_twiddle_a<XB, 1, INV, SAFE>(v, rare); break;
+    case 1:
+        if constexpr (XB >= 1) r16_twiddle_a<XB, 1, INV, SAFE>(v, rare);
+        break;
     case 2:
         if constexpr (XB == 2) r16_twiddle_a<XB, 2, INV, SAFE>(v, rare);
         break;
@@ -744,6 +751,11 @@ ZK_HD void r16_step_a(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, u
         if constexpr (XB == 2) r16_twiddle_a<XB, 3, INV, SAFE>(v, rare);
         break;
     default: break;
+    }
+    if constexpr (XB == 0) {
+        const u64 *tb = a.tb + 64 * v_;
+#pragma unroll
+        for (int kA = 1; kA < 16; kA++) v[kA] = f_mul<SAFE>(v[kA], tb[R::TS * kA], rare);
     }
     u64 *row = lds + g * R::GP + 16 * u + v_;
 #pragma unroll
@@ -781,10 +793,9 @@ ZK_HD void r16_role_c(const PassArgs &a, u32 tid, u32 &g, u32 &kA, u32 &kB)
     g = tid & (R::G - 1);
     kA = (tid >> R::GB) & 15;
     kB = tid >> (R::GB + 4);
-    if (XB == 1 && a.S == 0) {
-        const u32 x = g;
-        g = kA;
-        kA = x;
+    if (XB < 2 && a.S == 0) {  // a first pass: the wave's outputs of a group are contiguous
+        kA = tid & 15;
+        g = (tid >> 4) & (R::G - 1);
     }
 }
 
@@ -870,8 +881,9 @@ ZK_HD void r10_store(const PassArgs &a, u32 col, u64 jhi, u64 fast0, u32 tid, bo
 // workgroups per CU.
 inline u32 f10_gbits(const PassArgs &) { return 3; }
 
-// Groups per workgroup of the 9-bit form (log2).
+// Groups per workgroup of the 9-bit and 8-bit forms (log2).
 constexpr u32 kR9Gbits = R16<1>::GB;
+constexpr u32 kR8Gbits = R16<0>::GB;
 
 // The 16-element pass applies to 10-bit passes whose workgroup holds the
 // groups of one column: passes after the first, and first passes of
@@ -883,11 +895,22 @@ inline bool use_fast10(u32 B, const PassArgs &a)
     return B == 10 && extent >= (1ull << f10_gbits(a));
 }
 
-// Likewise the 9-bit form, for 9-bit passes whose fast dimension has its 16
-// groups.
+// Likewise the 9-bit and 8-bit forms, for passes whose fast dimension has
+// their 16 or 32 groups (9 bits: first pass 139 -> 106 us, second pass 176 ->
+// 140 us of a 57-column 2^19-point LDE).
 inline bool use_fast9(u32 B, const PassArgs &a)
 {
     return B == 9 && (a.S > 0 ? a.S : a.Jbits) >= kR9Gbits;
+}
+
+
+// First passes only: 2^23 x 4 columns 169 -> 134 us, 400 x 2^18 inverse 455 ->
+// 375 us, the first pass of 2^21-point LDEs 690 -> 595 us; later passes took 4
+// to 7 % longer than in the general kernel, whose 256 threads run each load
+// with its twiddle's.
+inline bool use_fast8(u32 B, const PassArgs &a)
+{
+    return B == 8 && a.S == 0 && a.Jbits >= kR8Gbits;
 }
 
 // Re-tiles a pass for the 16-element kernel: its groups per workgroup.
@@ -1036,11 +1059,13 @@ inline std::vector<PassPlan> plan_passes(const NttJob &job, const u64 *pw, const
         // first pass of a zero-extended input: the first L - lg_in DIT stages
         // of every step-A block only replicate
         a.skip = (S == 0 && fast) ? std::min<u32>(job.lg - job.lg_in, (B + 1) / 2) : 0;
-        PassPlan pp{a, B, ntiles, fast, false, false};
+        PassPlan pp{a, B, ntiles, fast, false, false, false};
         pp.r10 = fast && (!tune.np || tune.r10[p]) && use_fast10(B, a);
         if (pp.r10) f16_retile(pp, f10_gbits(a));
         pp.r9 = fast && (!tune.np || tune.r10[p]) && use_fast9(B, a);
         if (pp.r9) f16_retile(pp, kR9Gbits);
+        pp.r8 = fast && (!tune.np || tune.r10[p]) && use_fast8(B, a);
+        if (pp.r8) f16_retile(pp, kR8Gbits);
         out.push_back(pp);
         Sprev = S;
         S += B;
