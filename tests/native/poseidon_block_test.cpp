@@ -58,7 +58,7 @@ static void permute_hex(u64 st[12], bool &rare)
                 const u64 k = rc[12 * (r + 1) + (j < 12 ? j : j - 12)];
                 u64 x = (u32)k, y = k >> 32;
                 row_sum<0>(c[j].m, t, x, y);
-                s[j] = reduce_lohi42_nc(x, y, rare);
+                s[j] = reduce_lohi42(x, y);
             }
         }
     };
@@ -76,11 +76,11 @@ static void permute_hex(u64 st[12], bool &rare)
         }
         for (int q = 0; q < kBlock - 1; q++) {
             u64 v[16];
-            for (u32 j = 0; j < 16; j++) v[j] = reduce_lohi64(a[j], b[j], rare);
+            for (u32 j = 0; j < 16; j++) v[j] = reduce_lohi64_exact(a[j], b[j]);
             const u64 y = sbox_pair(v[12 + q], rare);
             for (u32 j = 0; j < 16; j++) row_add(c[j].b[12 + q], y, a[j], b[j]);
         }
-        for (u32 j = 0; j < 16; j++) s[j] = reduce_lohi64(a[j], b[j], rare);
+        for (u32 j = 0; j < 16; j++) s[j] = reduce_lohi64_exact(a[j], b[j]);
     }
     for (u32 e = 1; e < 12; e++) s[e] = gl_add_nc(s[e], rc[12 * 26 + e], rare);
     rounds(26, 30);
@@ -242,6 +242,7 @@ int main(int argc, char **argv)
         const u64 a = it % 4 ? g() % amax : amax - 1 - g() % 3, b = it % 4 ? g() % amax : amax - 1 - (g() % 3 << 31);
         bool rare = false;
         const u64 r = reduce_lohi64(a, b, rare);
+        expect("reduce_lohi64_exact", reduce_lohi64_exact(a, b), (u128)a % ZK_P + ((u128)(b % ZK_P) << 32) % ZK_P);
         if (!rare) expect("reduce_lohi64", r, (u128)a % ZK_P + ((u128)(b % ZK_P) << 32) % ZK_P);
         rare = false;
         const u64 c = a >> 22, d = b >> 22;

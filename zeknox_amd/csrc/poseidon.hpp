@@ -93,6 +93,19 @@ ZK_HD u64 reduce_lohi64(u64 a, u64 b, bool &rare)
     return ((u64)(hi + c2) << 32) | lo;
 }
 
+// The same with no rare case, the wraps entered as selected 2^32 - 1: three
+// instructions more, but none waits for a carry of the one before it.  Faster
+// where a wave runs alone (16 lanes per permutation: 7.17 -> 6.82 us), slower
+// at four waves per SIMD.
+ZK_HD u64 reduce_lohi64_exact(u64 a, u64 b)
+{
+    const u64 t = gl_reduce_small_mad_nc(a, (u32)(b >> 32));
+    unsigned c;
+    const u32 hi = __builtin_addc((u32)(t >> 32), (u32)b, 0u, &c);
+    const u64 r = ((u64)hi << 32) | (u32)t;
+    return r + (c ? ZK_EPS : 0);
+}
+
 // state <- M state + rcn (the next round's constants), M circulant (first row
 // circ) plus diag.  Row r is rcn[r] + sum of 13 products of a state element
 // with a constant below 2^6: the low and high 32-bit halves are accumulated

@@ -126,7 +126,7 @@ ZK_DEV void poseidon_permute_hex_nc(u64 &s, u32 j, const HexCoefs &c, bool &rare
             hex_gather(s, t);
             u64 a = (u32)rk, b = rk >> 32;
             row_sum<0>(c.m, t, a, b);
-            s = reduce_lohi42_nc(a, b, rare);
+            s = reduce_lohi42(a, b);
             rk = rk_next;
         }
     };
@@ -145,10 +145,10 @@ ZK_DEV void poseidon_permute_hex_nc(u64 &s, u32 j, const HexCoefs &c, bool &rare
         row_add(c.b[0], y, a, b);
         static_for<0, kBlock - 1>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            y = sbox7_pair(hex_bcast<12 + q>(reduce_lohi64(a, b, rare)), j & 1, LaneSwap(), rare);
+            y = sbox7_pair(hex_bcast<12 + q>(reduce_lohi64_exact(a, b)), j & 1, LaneSwap(), rare);
             row_add(c.b[12 + q], y, a, b);
         });
-        s = reduce_lohi64(a, b, rare);
+        s = reduce_lohi64_exact(a, b);
     }
     s = gl_add_nc(s, e ? rc[12 * 26 + e] : 0, rare);
     rounds(26, 30);
