@@ -50,17 +50,17 @@ struct PassPlan {
     u32 B;
     u64 ntiles;
     bool fast;
-    bool r10;  // runs the 16-element 10-bit kernel (ntt_r10_kernel)
-    bool r9;   // or its 9-bit form
-    bool r8;   // or its 8-bit form
+    bool r10;  // runs the 16-element kernel (ntt_r16_kernel<2>)
+    bool r9;   // or its 9-bit form (<1>)
+    bool r8;   // or its 8-bit form (<0>)
 };
 
 // Tuned plan of the transforms of one size 2^lg (lg <= 30), chosen by the
 // autotuner (zeknox_amd/tune.py) and loaded from its table when a device is
 // first used: the bits of each pass, each pass's groups per workgroup
-// (log2; kTuneAuto keeps the most the pass's extent and LDS allow) and, for
-// a 10-bit pass, whether the 16-element kernel may run it (else the
-// 32-element kernel does).  np == 0: no entry, the default plan.
+// (log2; kTuneAuto keeps the most the pass's extent and LDS allow) and, for a
+// 10-bit, 9-bit or first 8-bit pass, whether the 16-element kernel may run it
+// (else the general kernel does).  np == 0: no entry, the default plan.
 constexpr u32 kTuneAuto = 0xFFFFFFFFu;
 struct NttTune {
     u32 np;
