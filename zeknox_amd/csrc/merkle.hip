@@ -273,22 +273,38 @@ __global__ __launch_bounds__(kTreeNodeThreads) void level_hash_quad_kernel(u64 *
     }
 }
 
-// One level with 16 lanes per node (hash_two_hex), for levels whose latency
-// rather than their work bounds them.  Groups past the last node hash node 0
-// again and store nothing, so every group stays complete.
-__global__ __launch_bounds__(kTreeNodeThreads) void level_hash_hex_kernel(u64 *d, u64 nodes, u64 base, u64 n_sub,
-                                                                      u64 D)
+// Up to five consecutive levels with 16 lanes per node (hash_two_hex), for
+// levels whose latency rather than their work bounds them: a workgroup computes
+// 16 adjacent nodes of the first level (`nodes` per subtree, a multiple of 16)
+// and the nodes above them, passing digests on through LDS.  A launch for each
+// level cost 3 to 4 us more than its permutations' 7: the two levels of 2^11
+// and 2^10 nodes 24 -> 19 us, the four from 2^13 on 49 -> 39.  As in tree_top_kernel, a wave past the level's last node skips
+// it.
+constexpr u32 kChainNodes = 16;
+__global__ __launch_bounds__(16 * kChainNodes) void level_chain_hex_kernel(u64 *d, u64 nodes, u64 D, u32 levels)
 {
-    const u64 t = (u64)blockIdx.x * kTreeNodeThreads + threadIdx.x;
-    const u32 j = threadIdx.x & 15, lb = threadIdx.x & 48;  // lane in the group, group's first wave lane
-    const u64 total = nodes * n_sub, x = t >> 4;
-    const u64 xc = x < total ? x : 0;
-    const u64 s = xc / nodes, node = base + xc % nodes;
-    u64 *sd = d + s * D * 4;
+    __shared__ u64 buf[2][kChainNodes * 4];
+    const u64 x0 = (u64)blockIdx.x * kChainNodes;
+    u64 i0 = x0 % nodes;  // first node of the workgroup in its subtree's level
+    u64 *sd = d + x0 / nodes * D * 4;
+    const u32 j = threadIdx.x & 15, q = threadIdx.x >> 4, lb = threadIdx.x & 48;
+    const u32 wave_q0 = q & ~3u;  // the wave's first group
     HexCoefs c;
     hex_coefs(j, c);
-    const u64 out = hash_two_hex(sd + (2 * node + 2) * 4, sd + (2 * node + 3) * 4, j, lb, c);
-    if (x < total && j < 4) sd[node * 4 + j] = out;
+    for (u32 l = 0; l < levels; l++, nodes >>= 1, i0 >>= 1) {
+        const u32 count = kChainNodes >> l;
+        if (wave_q0 < count) {  // uniform across the wave
+            const u32 qc = q < count ? q : 0;
+            u64 *node = sd + (nodes - 2 + i0 + qc) * 4;
+            const u64 *ca = l ? buf[l & 1] + 8 * qc : sd + (2 * (nodes - 2 + i0 + qc) + 2) * 4;
+            const u64 h = hash_two_hex(ca, ca + 4, j, lb, c);
+            if (q < count && j < 4) {
+                node[j] = h;
+                buf[~l & 1][4 * q + j] = h;
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // One tree height of many commits in one launch (batched commits): G lanes
@@ -526,8 +542,8 @@ void merkle_launch(const TreeShape &t, u64 *digests, u64 *caps, const u64 *leave
     }
     if (nc == t.n_leaves) return;
     // Levels wider than the top kernel's: one lane per node while the level
-    // fills the GPU, a quad per node below that.  Level with r nodes per
-    // subtree starts at digest r - 2.
+    // fills the GPU, a quad per node below that, then 16 lanes and several
+    // levels a launch.  Level with r nodes per subtree starts at digest r - 2.
     const u64 m = std::min<u64>(L / 2, kTopNodes);
     for (u64 nodes = L / 2; nodes > m; nodes /= 2) {
         const u64 total = nodes * nc;
@@ -536,11 +552,17 @@ void merkle_launch(const TreeShape &t, u64 *digests, u64 *caps, const u64 *leave
             hipLaunchKernelGGL(level_hash_kernel, dim3(blocks_for(total, kTreeNodeThreads)), dim3(kTreeNodeThreads), 0, st,
                                digests, nodes, nodes - 2, nc, D);
         else if (total > kHexMaxNodes)
-            hipLaunchKernelGGL(level_hash_quad_kernel, dim3(blocks_for(4 * total, kTreeNodeThreads)), dim3(kTreeNodeThreads),
-                               0, st, digests, nodes, nodes - 2, nc, D);
-        else
-            hipLaunchKernelGGL(level_hash_hex_kernel, dim3(blocks_for(16 * total, kTreeNodeThreads)), dim3(kTreeNodeThreads),
-                               0, st, digests, nodes, nodes - 2, nc, D);
+            hipLaunchKernelGGL(level_hash_quad_kernel, dim3(blocks_for(4 * total, kTreeNodeThreads)),
+                               dim3(kTreeNodeThreads), 0, st, digests, nodes, nodes - 2, nc, D);
+        else {
+            // the levels from here to the top's, up to five a launch (every
+            // level here has more than kTopNodes nodes per subtree)
+            u32 levels = 1;
+            while (levels < 5 && nodes >> levels > m) levels++;
+            hipLaunchKernelGGL(level_chain_hex_kernel, dim3((u32)(total / kChainNodes)), dim3(16 * kChainNodes), 0, st,
+                               digests, nodes, D, levels);
+            nodes >>= levels - 1;
+        }
         ZK_HIP(hipGetLastError());
     }
     ProfScope ps("merkle.top", st);
