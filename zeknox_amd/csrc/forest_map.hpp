@@ -21,12 +21,12 @@ namespace zk {
 constexpr int kLeafThreads = 128;  // threads per workgroup of the forests' leaf kernels
 constexpr int kNodeThreads = 128;  // threads per workgroup of the forests' level kernels
 // Levels with at most this many nodes (all subtrees) use a quad of lanes per
-// node: 36 us at 2^16 nodes against 39 with one lane; at 2^17 one lane takes
-// 53 us, a quad 70.
+// node: 35 us at 2^16 nodes against 38 with one lane; at 2^17 one lane takes
+// 52 us, a quad 70.
 constexpr u64 kQuadMaxNodes = 1u << 16;
-// Levels with at most this many nodes use 16 lanes per node: 11 us at 2^13
-// nodes against 13 with a quad, 7.7 at 2^12; at 2^14 a quad takes 13 us, 16
-// lanes 20.
+// Levels with at most this many nodes use 16 lanes per node: 10 us at 2^13
+// nodes against 12.3 with a quad, 6.8 at 2^12; at 2^14 a quad takes 12.3 us, 16
+// lanes 18.
 constexpr u64 kHexMaxNodes = 1u << 13;
 // Workgroups of one forest launch at most (HIP counts a grid in threads, as a
 // 32-bit number); a longer launch is split, each part with its own table.

@@ -27,8 +27,8 @@ namespace zk {
 
 // Lanes per leaf by the number of leaves, where one form's time per
 // permutation passes the other's on an MI355X (1024 SIMDs): 16 lanes up to
-// 2^13 leaves (two waves per SIMD: 10.9 us; a quad 13.1), a quad up to 2^16
-// (19 us at 2^15, 36 at 2^16; one lane 39 at either), then one lane (53 us at
+// 2^13 leaves (two waves per SIMD: 10 us; a quad 12.3), a quad up to 2^16
+// (18 us at 2^15, 35 at 2^16; one lane 38 at either), then one lane (52 us at
 // 2^17, where a quad takes 70).
 constexpr u64 kHexMaxLeaves = 1u << 13;
 constexpr u64 kQuadMaxLeaves = 1u << 16;
@@ -278,8 +278,9 @@ __global__ __launch_bounds__(kTreeNodeThreads) void level_hash_quad_kernel(u64 *
 // 16 adjacent nodes of the first level (`nodes` per subtree, a multiple of 16)
 // and the nodes above them, passing digests on through LDS.  A launch for each
 // level cost 3 to 4 us more than its permutations' 7: the two levels of 2^11
-// and 2^10 nodes 24 -> 19 us, the four from 2^13 on 49 -> 39.  As in tree_top_kernel, a wave past the level's last node skips
-// it.
+// and 2^10 nodes 24 -> 19 us, all levels of a tree of 2^15 leaves 73 -> 66 (the
+// four from 2^13 nodes on take 40).  As in tree_top_kernel, a wave past the
+// level's last node skips it.
 constexpr u32 kChainNodes = 16;
 __global__ __launch_bounds__(16 * kChainNodes) void level_chain_hex_kernel(u64 *d, u64 nodes, u64 D, u32 levels)
 {
