@@ -110,6 +110,12 @@ static std::vector<u64> transform(u32 lg, u32 lg_in, u32 ncols, bool inv, bool c
                 tws.back()[i] = twiddle_entry(pw[inv].data(), pp.a.L, pp.a.S, pp.a.Sprev, i);
             pp.a.tw = tws.back().data();
         }
+        // the rule takes the 8-bit form for launches that fill the chip; its
+        // arithmetic is run here on small ones
+        if (r9 && pp.B == 8 && pp.a.S == 0 && pp.a.Jbits >= kR8Gbits && !pp.r8) {
+            pp.r8 = true;
+            f16_retile(pp, kR8Gbits);
+        }
         nr9 += pp.r9 || pp.r8;
         inv ? run_pass<true>(pp) : run_pass<false>(pp);
     }

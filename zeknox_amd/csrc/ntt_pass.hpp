@@ -903,14 +903,16 @@ inline bool use_fast9(u32 B, const PassArgs &a)
     return B == 9 && (a.S > 0 ? a.S : a.Jbits) >= kR9Gbits;
 }
 
-
 // First passes only: 2^23 x 4 columns 169 -> 134 us, 400 x 2^18 inverse 455 ->
 // 375 us, the first pass of 2^21-point LDEs 690 -> 595 us; later passes took 4
 // to 7 % longer than in the general kernel, whose 256 threads run each load
-// with its twiddle's.
+// with its twiddle's.  From 2^18 points on and with a workgroup for each of the
+// kernel's 512 slots (whole transforms of 2^18 points: 16 columns 61 -> 58 us, 1
+// column 34.7 -> 35.2; of 2^16 points 1 column 28.3 -> 30.0, 64 columns 56.7 ->
+// 58.7: a launch of one round is latency, and smaller workgroups spread better).
 inline bool use_fast8(u32 B, const PassArgs &a)
 {
-    return B == 8 && a.S == 0 && a.Jbits >= kR8Gbits;
+    return B == 8 && a.S == 0 && a.Jbits >= 10 && ((u64)a.ncols << (a.Jbits - kR8Gbits)) >= 512;
 }
 
 // Re-tiles a pass for the 16-element kernel: its groups per workgroup.
