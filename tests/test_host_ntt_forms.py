@@ -70,3 +70,22 @@ def test_forms_equal_oracle(harness, tmp_path, lg, lg_in, C, inv, coset, force, 
     else:
         ref = O.lde(x, lg_in, lg - lg_in, C, inverse=bool(inv), with_coset=bool(coset))
     assert (got == ref).all(), r.stdout
+
+
+@pytest.mark.parametrize("bits,C,want", [
+    ((8, 10), 15, "general"), ((8, 10), 16, "r8"),          # 512 workgroups
+    ((8, 7, 7), 1, "r8"),                                   # 2^22: no other 8-bit pass
+    ((8, 5, 8), 11, "general"), ((8, 5, 8), 12, "r8"),      # 3072 workgroups where a later pass has 8 bits
+    ((8, 8, 7), 2, "general"), ((8, 8, 7), 3, "r8"),
+    ((8, 8, 8), 1, "general"), ((8, 8, 8), 2, "r8"),
+    ((8, 8), 400, "general"),                               # 2^16
+])
+def test_where_a_first_8bit_pass_takes_its_form(harness, bits, C, want):
+    """An 8-bit first pass beside another 8-bit pass stays on the general
+    kernel, whose code that pass runs too, until the launch is large."""
+    lg = sum(bits)
+    r = subprocess.run([harness, str(lg), str(lg), str(C), "0", "0", "0", "0", "-", "-"] + plan_args(bits),
+                       capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr
+    got = forms(r.stdout)
+    assert got[0] == want and "r8" not in got[1:], r.stdout

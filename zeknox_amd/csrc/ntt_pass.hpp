@@ -910,9 +910,18 @@ inline bool use_fast9(u32 B, const PassArgs &a)
 // kernel's 512 slots (whole transforms of 2^18 points: 16 columns 61 -> 58 us, 1
 // column 34.7 -> 35.2; of 2^16 points 1 column 28.3 -> 30.0, 64 columns 56.7 ->
 // 58.7: a launch of one round is latency, and smaller workgroups spread better).
-inline bool use_fast8(u32 B, const PassArgs &a)
+// `again`: a later pass has 8 bits too.  It runs the general kernel, whose
+// instructions are at hand when the first pass ran it as well; else it takes 3
+// to 4 us longer (2^21 as 8 + 5 + 8 bits, 2 columns: 25.4 -> 29.0; as 8 + 7 + 6
+// no such step), more than the first pass gains while the data stay in the
+// 256 MiB cache.  So such plans need 3072 workgroups, 1.5 x 2^24 elements:
+// whole transforms of 2^21 points x 3 columns 97.0 -> 101.0 us, x 12 328 -> 321;
+// 2^23 x 1 130 -> 133, x 2 221 -> 224, x 3 357 -> 345; 2^24 x 1 212 -> 216, x 2
+// 456 -> 432; LDEs of 2^21 points x 10 228 -> 231, x 16 384 -> 382.
+inline bool use_fast8(u32 B, const PassArgs &a, bool again)
 {
-    return B == 8 && a.S == 0 && a.Jbits >= 10 && ((u64)a.ncols << (a.Jbits - kR8Gbits)) >= 512;
+    return B == 8 && a.S == 0 && a.Jbits >= 10 &&
+           ((u64)a.ncols << (a.Jbits - kR8Gbits)) >= (again ? 3072u : 512u);
 }
 
 // Re-tiles a pass for the 16-element kernel: its groups per workgroup.
@@ -1066,7 +1075,7 @@ inline std::vector<PassPlan> plan_passes(const NttJob &job, const u64 *pw, const
         if (pp.r10) f16_retile(pp, f10_gbits(a));
         pp.r9 = fast && (!tune.np || tune.r10[p]) && use_fast9(B, a);
         if (pp.r9) f16_retile(pp, kR9Gbits);
-        pp.r8 = fast && (!tune.np || tune.r10[p]) && use_fast8(B, a);
+        pp.r8 = fast && (!tune.np || tune.r10[p]) && use_fast8(B, a, std::count(bits + p + 1, bits + np, 8u) > 0);
         if (pp.r8) f16_retile(pp, kR8Gbits);
         out.push_back(pp);
         Sprev = S;
