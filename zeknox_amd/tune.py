@@ -4,9 +4,10 @@ For every transform size 2^lg it runs the coset LDE of the commit path (135
 columns, blowup 8: 2^(lg-3) coefficients per column -> 2^lg rows) under each
 candidate plan -- the split of the lg bits into 1..3 HBM passes of at most 10
 bits, the groups per workgroup of the passes (the tile width: more groups make
-longer contiguous row runs and use more LDS), and for a 10-bit pass the
-16-element kernel (512 threads, 8 groups, a 16 x 4 x 16 split) or the
-32-element kernel (two 32-point register DITs, more LDS per group) -- checks
+longer contiguous row runs and use more LDS), and for the 10-bit and 9-bit
+passes and a first 8-bit pass the 16-element kernel (512 threads, 8, 16 or 32
+groups, a 16 x 4 x 16, 16 x 2 x 16 or 16 x 16 split; it has that one tile width)
+or the general kernel (two register DITs of up to 32 points) -- checks
 that the output equals the default plan's bit for bit, times the passes with
 the library's per-kernel HIP-event timings (median of --reps runs), and writes
 the fastest plan of each size to the table the library loads when a device is
@@ -55,14 +56,23 @@ def splits(lg):
     return out
 
 
+def kernel16_options(bits):
+    """16-element kernel flags to try for a split: allowed everywhere, and the
+    general kernel instead for the passes of one of its sizes (10 bits, 9 bits,
+    8 bits in the first pass; the flag has no meaning for other passes)."""
+    opts = [(1,) * len(bits)]
+    for size in (10, 9, 8):
+        off = tuple(int(b != size or (size == 8 and p > 0)) for p, b in enumerate(bits))
+        if 0 in off and (size == 10 or len(bits) > 1):
+            opts.append(off)
+    return opts
+
+
 def candidates(lg):
     seen = set()
     for bits in splits(lg):
-        k16_opts = [(1,) * len(bits)]
-        if 10 in bits:
-            k16_opts.append(tuple(0 if b == 10 else 1 for b in bits))
         for g in GBITS:
-            for k16 in k16_opts:
+            for k16 in kernel16_options(bits):
                 plan = (bits, (g,) * len(bits), k16)
                 if plan not in seen:
                     seen.add(plan)
@@ -148,7 +158,8 @@ def write_table(results, path, C, reps):
              % reps,
              "# default three times round-robin (best median each); written %s." % time.strftime("%Y-%m-%d"),
              "# lg np b1 b2 b3 g1 g2 g3 k1 k2 k3   (b: bits per pass, g: log2 groups per workgroup, -1 the most",
-             "# the pass allows, k: 1 = the 16-element kernel may run a 10-bit pass)"]
+             "# the pass allows, k: 1 = the 16-element kernel may run a 10-bit, 9-bit or first 8-bit pass, with its",
+             "# own number of groups)"]
     for lg, t_def, t_best, chosen in results:
         if chosen is None:
             lines.append("# %d default %s %.4f ms (no plan measured %.0f%% faster)" % (
