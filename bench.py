@@ -52,8 +52,8 @@ HBM_PEAK = 8.0e12  # MI355X HBM3E, bytes/s
 # second.  The leaf-hash roofline's peak is the issue-limited rate of the
 # library's own permutation on this part: the leaf kernel's sponge with its
 # inputs computed in registers, no memory traffic, as many waves per SIMD as
-# the registers allow (tests/native/perm_rate.hip, result kept in the traffic
-# profile); the SIMD-cycles per wave-permutation it measures are reported
+# the registers allow (tests/native/perm_rate_mfma.hip, result kept in the
+# traffic profile); the SIMD-cycles per wave-permutation it measures are reported
 # beside it.
 SIMD_CYCLES_PER_S = 256 * 4 * 2.4e9
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "commit_135x2p20_traffic.json")

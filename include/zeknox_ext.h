@@ -141,7 +141,8 @@ RustError zk_server_destroy(zk_server *server);
  * split into 1..3 HBM passes of at most 10 bits (bits[0..npasses)), each
  * pass's groups per workgroup (gbits, log2; -1: the most the pass allows)
  * and, for a 10-bit, 9-bit or first 8-bit pass, whether the 16-element kernel
- * may run it (kernel16 = 1) or the general kernel does (0).  The autotuner
+ * may run it (kernel16 = 1) or the general kernel does (0); the 16-element
+ * kernel has its own number of groups and ignores gbits.  The autotuner
  * (zeknox_amd/tune.py) measures candidate plans per size and writes the best
  * to ntt_tuning_gfx950.txt beside the library, which is loaded when a device
  * is first used (ZK_NTT_TUNING names another file).  Every plan computes the

@@ -2,11 +2,11 @@
 // form with the full rounds' layers on the matrix cores; perm_rate.hip is the
 // multiply-add form): every lane runs the leaf kernel's sponge (hash_one) over a 135-element leaf whose
 // elements it computes from its index (no memory traffic but the digest
-// store), launched in the leaf-hash kernel's shape
-// (workgroups of 128 lanes, at least four waves per SIMD, 2^20 lanes), so the
+// store), launched over 2^20 lanes at the leaf kernels' four waves per SIMD
+// (workgroups of 128 lanes, as the forests'; a single tree's have 256), so the
 // rate is what the permutation's instruction stream reaches when nothing but
 // VALU issue limits it, with as many waves per SIMD as the registers allow
-// and, for comparison, with four or five (capped through LDS).  bench.py's
+// and, for comparison, with their placement limited through LDS.  bench.py's
 // leaf-hash roofline divides the leaf kernel's permutation rate by the first.  Prints permutations per second and
 // SIMD-cycles per wave-permutation (256 CUs x 4 SIMDs at 2.4 GHz).
 //
@@ -22,8 +22,8 @@ using namespace zk;
 constexpr int kThreads = 128;
 constexpr int kPerms = 17;  // permutations per lane: a 135-element leaf
 
-// LDS bytes per workgroup caps the waves per SIMD (160 KiB per CU, two waves
-// per workgroup): 0 leaves the register count as the only limit.
+// LDS bytes per workgroup limit the workgroups per CU (160 KiB): 0 leaves the
+// register count as the only limit.
 template <u32 LDS_BYTES>
 __global__ __launch_bounds__(kThreads, 4) void perm_rate_kernel(u64 *out, u64 seed)
 {
@@ -80,11 +80,10 @@ int main()
     const u32 lanes = 1u << 20;
     u64 *out = nullptr;
     if (hipMalloc(&out, (size_t)lanes * sizeof(u64)) != hipSuccess) return 1;
-    // registers only; LDS-capped to five and four waves per SIMD (10 and 8
-    // workgroups per CU)
+    // registers only (four waves per SIMD); LDS for 10 and 8 workgroups per CU
     int rc = run<0>(out, lanes, "registers only");
-    rc |= run<16384>(out, lanes, "5 waves per SIMD");
-    rc |= run<20480>(out, lanes, "4 waves per SIMD");
+    rc |= run<16384>(out, lanes, "10 workgroups per CU");
+    rc |= run<20480>(out, lanes, "8 workgroups per CU");
     (void)hipFree(out);
     return rc;
 }

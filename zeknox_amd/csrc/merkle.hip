@@ -83,8 +83,7 @@ __device__ __forceinline__ u64 *leaf_out(const LeafArgs &a, u64 leaf)
 // them: in the leaf kernel a copy waits for the permutation's tables (16 loads
 // a lane) and runs at its four waves per SIMD.  Trees that are all caps, 1
 // element: 2^10 leaves 13.8 -> 12.8 us, 2^20 25.0 -> 20.9.  (The forests' leaf
-// kernel keeps both: with the copy as a branch before the tables it took 3 %
-// longer for the leaves that are hashed.)
+// kernel keeps both, as one launch holds jobs of either kind.)
 template <LeafLayout LAYOUT, bool ROWS>
 __global__ __launch_bounds__(kTreeLeafThreads) void leaf_copy_kernel(LeafArgs a)
 {

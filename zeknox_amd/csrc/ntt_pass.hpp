@@ -59,8 +59,9 @@ struct PassPlan {
 // autotuner (zeknox_amd/tune.py) and loaded from its table when a device is
 // first used: the bits of each pass, each pass's groups per workgroup
 // (log2; kTuneAuto keeps the most the pass's extent and LDS allow) and, for a
-// 10-bit, 9-bit or first 8-bit pass, whether the 16-element kernel may run it
-// (else the general kernel does).  np == 0: no entry, the default plan.
+// 10-bit, 9-bit or first 8-bit pass, whether the 16-element kernel may run it,
+// with its own groups (else the general kernel does).  np == 0: no entry, the
+// default plan.
 constexpr u32 kTuneAuto = 0xFFFFFFFFu;
 struct NttTune {
     u32 np;
@@ -168,8 +169,8 @@ struct Pass {
     // blocks across all columns: the tiles that run together on one XCD
     // (about 64) cover 8 columns x 8 adjacent fast blocks, so their rows are
     // read and written in 512-byte runs and they share one slice of the
-    // twiddle table in L2.  Wider tiles (whose rows are already 512-byte
-    // runs) take the fast index fastest.
+    // twiddle table in L2.  Wider tiles (rows of 128 to 512 bytes) take the
+    // fast index fastest, which measured faster for 7-bit passes.
     ZK_HD static void tile_decode(const PassArgs &a, u64 t, u32 &col, u64 &jhi, u64 &fast0)
     {
         if (a.S > 0 && a.Gbits > 3) {
@@ -896,8 +897,9 @@ inline bool use_fast10(u32 B, const PassArgs &a)
 }
 
 // Likewise the 9-bit and 8-bit forms, for passes whose fast dimension has
-// their 16 or 32 groups (9 bits: first pass 139 -> 106 us, second pass 176 ->
-// 140 us of a 57-column 2^19-point LDE).
+// their 16 or 32 groups (9 bits, LDE of 57 columns to 2^19 points: first pass of
+// 9 + 10 bits, the plan it has, 139 -> 106 us; second pass of 10 + 9 bits 176 -> 140
+// us.  9-bit passes after the first are in the default plans of 2^26 and 2^27).
 inline bool use_fast9(u32 B, const PassArgs &a)
 {
     return B == 9 && (a.S > 0 ? a.S : a.Jbits) >= kR9Gbits;
@@ -912,9 +914,9 @@ inline bool use_fast9(u32 B, const PassArgs &a)
 // 58.7: a launch of one round is latency, and smaller workgroups spread better).
 // `again`: a later pass has 8 bits too.  It runs the general kernel, whose
 // instructions are at hand when the first pass ran it as well; else it takes 3
-// to 4 us longer (2^21 as 8 + 5 + 8 bits, 2 columns: 25.4 -> 29.0; as 8 + 7 + 6
-// no such step), more than the first pass gains while the data stay in the
-// 256 MiB cache.  So such plans need 3072 workgroups, 1.5 x 2^24 elements:
+// to 4 us longer (2^21 points x 2 columns, the last 8 bits: 25 us after 8 + 5 or
+// 5 + 8 in the general kernel, 29 after 7 + 6, 9 + 4 or 8 + 5 with this form
+// first), more than the first pass gains while the data stay in the 256 MiB cache.  So such plans need 3072 workgroups, 1.5 x 2^24 elements:
 // whole transforms of 2^21 points x 3 columns 97.0 -> 101.0 us, x 12 328 -> 321;
 // 2^23 x 1 130 -> 133, x 2 221 -> 224, x 3 357 -> 345; 2^24 x 1 212 -> 216, x 2
 // 456 -> 432; LDEs of 2^21 points x 10 228 -> 231, x 16 384 -> 382.

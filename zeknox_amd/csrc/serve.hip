@@ -11,8 +11,8 @@
 // (forest_launch_tables: one leaf-hash launch over every leaf of the group and
 // one launch per tree height, as the batched commits do), followed by the cap
 // copies and one event per request.  A group of one request runs the single-
-// commit kernels instead (commit_launch: quad-lane leaves and tree tops for
-// small trees, which cut its latency).  Groups admitted while others run
+// commit kernels instead (commit_launch: 16 lanes or a quad per leaf and
+// chained levels for small trees, which cut its latency).  Groups admitted while others run
 // overlap with them on the device.  The worker polls the events, copies each
 // finished cap out of a pinned staging slot, returns the memory (unless the
 // caller keeps the LDE and digests resident for openings) and admits whatever
